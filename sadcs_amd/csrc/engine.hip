@@ -32,6 +32,7 @@
 #include "merge.h"
 #include "prim.h"
 #include "rank.h"
+#include "small.h"
 
 namespace sadcs {
 
@@ -411,6 +412,7 @@ struct Params {
     uint32_t g = defaultSplitterSpacing(32);  // splitter spacing
     uint32_t k = 0;                           // sorted splitters per tile; 0: the most that keep the CU's tiles in its LDS
     int threads = defaultTileThreads(32);     // threads per merge tile (512 or 256)
+    bool tiles = false;                       // merge parameters given: every build takes the tile merge
 
     // Zero fields take the defaults of the cover.
     void apply(const sadcs_params* p) {
@@ -422,6 +424,7 @@ struct Params {
         if (p && p->tile_splitters) {
             k = p->tile_splitters;
         }
+        tiles = p && (p->splitter_spacing || p->tile_splitters || p->tile_threads);
     }
 };
 
@@ -2216,8 +2219,153 @@ int buildWith(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, Text
     return SADCS_OK;
 }
 
+// ---- small texts: one workgroup each --------------------------------------------------------------
+
+// A host call whose text (or outputs) fit this many bytes passes them through the pinned staging
+// chunks, which the kernel reads and writes itself: a DMA's own latency is longer.
+constexpr size_t kZeroCopyBytes = size_t(1) << 18;
+
+template <int kThreads, int kItems>
+int launchSmallTexts(hipStream_t stream, uint32_t texts, const uint8_t* text, const Segment* segments, uint32_t capacity, uint32_t* sa, uint8_t* bwt, uint32_t* firstRows, uint32_t* rounds) {
+    const auto kernel = smallTextsKernel<kThreads, kItems>;
+    const size_t shared = smallSharedBytes(capacity, kThreads);
+    SADCS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(shared)));
+    kernel<<<texts, kThreads, shared, stream>>>(text, segments, capacity, sa, bwt, firstRows, rounds);
+    SADCS_HIP(hipGetLastError());
+    return SADCS_OK;
+}
+
+// Whether buildSmall takes a build: short texts, SA and/or BWT, no merge parameters given (those
+// ask for the tile merge), and room for the tables in the pinned chunks.
+bool isSmall(const sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq) {
+    return layout.maxLength <= kSmallMax && rq.mode != Mode::RankOnly && !ctx.params.tiles && ctx.staging[0] && ctx.staging[1] &&
+           layout.segments.size() * (sizeof(Segment) + sizeof(uint32_t)) + 4096 <= kStagingChunk / 2;
+}
+
+int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sadcs_stats* stats) {
+    Arena& arena = ctx.arena;
+    arena.reset(ctx.arenaBase, ctx.arenaBytes, false);
+    const bool deviceCall = rq.deviceText != nullptr;
+    const bool wantSA = rq.mode != Mode::BWT, wantBWT = rq.mode != Mode::SA;
+    const size_t count = layout.segments.size();
+    const size_t total = static_cast<size_t>(layout.totalLength);
+
+    // Chunk 1 holds the segment table, the first rows and the rounds; then small outputs.
+    SADCS_HIP(hipStreamSynchronize(ctx.stream));
+    Segment* segments = reinterpret_cast<Segment*>(ctx.staging[1]);
+    uint32_t* firstRows = reinterpret_cast<uint32_t*>(segments + count);
+    uint32_t* rounds = firstRows + count;
+    std::copy(layout.segments.begin(), layout.segments.end(), segments);
+    *rounds = 0;
+    const size_t tableBytes = (count * (sizeof(Segment) + sizeof(uint32_t)) + sizeof(uint32_t) + 255) / 256 * 256;
+
+    const auto uploadStart = std::chrono::steady_clock::now();
+    const uint8_t* text = rq.deviceText;
+    bool pinned = false;
+    if (!deviceCall) {
+        pinned = true;
+        const size_t span = layout.span;
+        auto each = [&](auto put) {
+            const uint8_t* src = rq.hostText;
+            for (size_t i = 0; i < count; i++) {
+                const size_t n = layout.segments[i].end - layout.segments[i].start;
+                put(layout.segments[i].start, rq.hostTexts ? rq.hostTexts[i] : src, n);
+                src += n;
+            }
+        };
+        if (span <= kStagingChunk) {
+            each([&](size_t at, const uint8_t* src, size_t n) { memcpy(ctx.staging[0] + at, src, n); });
+            text = ctx.staging[0];
+        }
+        if (span > kZeroCopyBytes) {
+            uint8_t* device = nullptr;
+            SADCS_TRY(arena.allocate(device, span));
+            if (span <= kStagingChunk) {
+                SADCS_HIP(hipMemcpyAsync(device, ctx.staging[0], span, hipMemcpyHostToDevice, ctx.stream));
+            } else {
+                int status = SADCS_OK;
+                each([&](size_t at, const uint8_t* src, size_t n) {
+                    status = status == SADCS_OK ? static_cast<int>(hipMemcpyAsync(device + at, src, n, hipMemcpyHostToDevice, ctx.stream) == hipSuccess ? SADCS_OK : SADCS_FAILED) : status;
+                });
+                if (status != SADCS_OK) {
+                    setError("upload of small texts failed");
+                    return status;
+                }
+            }
+            text = device;
+        }
+    }
+    const double uploadSeconds = deviceCall ? 0 : secondsSince(uploadStart);
+
+    uint32_t* sa = wantSA ? rq.deviceSA : nullptr;
+    uint8_t* bwt = wantBWT ? rq.deviceBWT : nullptr;
+    const bool zeroCopyOut = !deviceCall && total * 5 <= kZeroCopyBytes && tableBytes + total * 5 + 256 <= kStagingChunk;
+    if (zeroCopyOut) {
+        sa = wantSA ? reinterpret_cast<uint32_t*>(ctx.staging[1] + tableBytes) : nullptr;
+        bwt = wantBWT ? ctx.staging[1] + tableBytes + total * sizeof(uint32_t) : nullptr;
+    } else if (!deviceCall) {
+        if (wantSA) SADCS_TRY(arena.allocate(sa, total));
+        if (wantBWT) SADCS_TRY(arena.allocate(bwt, total));
+    }
+
+    const auto deviceStart = std::chrono::steady_clock::now();
+    const uint32_t capacity = (layout.maxLength + 63) / 64 * 64;
+    const uint32_t texts = static_cast<uint32_t>(count);
+    if (capacity <= 2048) {
+        SADCS_TRY((launchSmallTexts<256, 16>(ctx.stream, texts, text, segments, capacity, sa, bwt, firstRows, rounds)));
+    } else {
+        SADCS_TRY((launchSmallTexts<1024, 32>(ctx.stream, texts, text, segments, capacity, sa, bwt, firstRows, rounds)));
+    }
+    SADCS_HIP(hipStreamSynchronize(ctx.stream));
+    const double deviceSeconds = secondsSince(deviceStart);
+
+    if (wantBWT && rq.hostPrimaries) {
+        for (size_t i = 0; i < count; i++) {
+            rq.hostPrimaries[i] = static_cast<int32_t>(firstRows[i]) + 1;
+        }
+    }
+    PhaseTimes times;
+    times.merge = deviceSeconds;  // one kernel does all the phases
+    times.mergeKernel = deviceSeconds;
+    times.mergeElements = layout.totalLength;
+    times.characterPasses = 1;
+    times.doublingRounds = static_cast<int>(*rounds);
+    times.rankingBytes = times.classBytes = times.mergeBytes = arena.highWater();
+    const auto downloadStart = std::chrono::steady_clock::now();
+    if (!deviceCall) {
+        if (wantSA && rq.hostSA) {
+            if (zeroCopyOut) {
+                memcpy(rq.hostSA, sa, total * sizeof(uint32_t));
+            } else {
+                SADCS_TRY(download(ctx, rq.hostSA, sa, total * sizeof(uint32_t)));
+            }
+        }
+        if (wantBWT && rq.hostBWT) {
+            if (zeroCopyOut) {
+                memcpy(rq.hostBWT, bwt, total);
+            } else {
+                SADCS_TRY(download(ctx, rq.hostBWT, bwt, total));
+            }
+        }
+    }
+    size_t deviceBytes = arena.highWater();
+    if (deviceCall) {
+        deviceBytes += static_cast<size_t>(layout.span) + kTextPadding + (wantSA ? total * 4 : 0) + (wantBWT ? total : 0);
+    }
+    fillStats(stats, times, deviceBytes, ctx.params.cover);
+    if (stats) {
+        stats->upload_seconds = uploadSeconds;
+        stats->pinned = pinned ? 1 : 0;
+        stats->download_seconds = secondsSince(downloadStart);
+    }
+    return SADCS_OK;
+}
+
 int build(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sadcs_stats* stats) {
     (void)hipGetLastError();  // errors of earlier, unrelated calls are not this construction's
+    if (isSmall(ctx, layout, rq)) {
+        return buildSmall(ctx, layout, rq, stats);
+    }
     const bool batch = !layout.blockSegment.empty();
     if (ctx.params.cover == 128) {
         return batch ? buildWith<128, TextBatch>(ctx, layout, rq, TextBatch{}, stats)
