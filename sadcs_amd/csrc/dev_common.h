@@ -65,14 +65,19 @@ __device__ __forceinline__ uint64_t ballot(bool predicate) {
 // Lanes of the wave that are valid and hold the same BITS-bit digit as this lane.
 template <int BITS>
 __device__ __forceinline__ uint64_t matchDigit(uint32_t digit, bool valid) {
-    uint64_t peers = ballot(valid);
+    // Per bit, lanes agree with this one where the ballot equals its own bit spread over a word: one
+    // extract, one compare and two three-input bit operations, against seven instructions with
+    // selects of the ballot and its complement.
+    const uint64_t all = ballot(valid);
+    uint32_t lo = static_cast<uint32_t>(all), hi = static_cast<uint32_t>(all >> 32);
 #pragma unroll
     for (int b = 0; b < BITS; b++) {
-        const bool bit = (digit >> b) & 1;
-        const uint64_t set = ballot(bit);
-        peers &= bit ? set : ~set;
+        const uint32_t own = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(digit), b, 1));
+        const uint64_t set = ballot(own != 0);
+        lo &= ~(static_cast<uint32_t>(set) ^ own);
+        hi &= ~(static_cast<uint32_t>(set >> 32) ^ own);
     }
-    return peers;
+    return static_cast<uint64_t>(hi) << 32 | lo;
 }
 
 // ---- wave scans on DPP --------------------------------------------------------------------------

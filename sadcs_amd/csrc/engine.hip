@@ -30,6 +30,7 @@
 #include "cover.h"
 #include "dev_common.h"
 #include "merge.h"
+#include "prefix.h"
 #include "prim.h"
 #include "rank.h"
 #include "small.h"
@@ -255,6 +256,10 @@ class Arena {
         return m_highWater;
     }
 
+    size_t live() const {
+        return m_live;
+    }
+
     void resetHighWater() {
         size_t top = 0;
         for (const Block& b : m_used) {
@@ -448,6 +453,8 @@ struct Job {
     int32_t* hostSA = nullptr;              // host calls: where the outputs go; the merge
     uint8_t* hostBWT = nullptr;             //   downloads them as it finishes slices of rows
     bool downloaded = false;                //   and sets this when it has
+    bool alphabetKnown = false;             // the bytes that occur, once read back
+    uint32_t alphabetMask[8] = {};
 };
 
 // The outputs of a top-level merge in slices, for downloadSlices: rows[0] = 0 < ... <
@@ -485,6 +492,7 @@ struct sadcs_ctx {
     uint8_t* arenaBase = nullptr;
     size_t arenaBytes = 0;
     sadcs::Arena arena;
+    size_t budget = 0;                 // device bytes this call may use of the arena; 0: all of it
     uint32_t* hostWords = nullptr;     // pinned, for readbacks
     uint8_t* staging[2] = {};          // pinned staging chunks
     hipEvent_t stagingDone[2] = {};
@@ -501,16 +509,16 @@ struct sadcs_ctx {
 namespace sadcs {
 
 constexpr size_t kStagingChunk = size_t(32) << 20;
-// Pinned readback words: [0, 264) the text's byte presence (at the start of ranking), [0, 16)
-// counters, [16, 1016) the first rows of a batch (after the build), [kSliceRowWords, +kSlices + 1)
+// Pinned readback words: [0, 2050) the prefix sort's bucket rows, [0, 16) counters, [16, 1016) the first rows of a batch (after the build), [kSliceRowWords, +kSlices + 1)
 // the row bounds of the top-level merge's slices.
-constexpr size_t kHostWords = 2048;
+constexpr size_t kHostWords = 4096;
 constexpr size_t kSliceRowWords = 1024;
 // The top-level merge of a host call is launched in slices of about this many output rows (at
 // most sadcs_ctx::kSlices), so the download of finished rows overlaps the rest of the merge.
 constexpr uint64_t kSliceRows = uint64_t(1) << 24;
 constexpr int64_t kMemoryReserve = int64_t(256) << 20;
 constexpr size_t kTextPadding = 64;
+constexpr size_t kFreeBudget = size_t(256) << 20;
 
 bool gTablesReady[2] = {false, false};
 
@@ -581,10 +589,7 @@ class Pipeline {
         m_g = ctx.params.g;
         m_threads = ctx.params.threads;
         m_k = ctx.params.k ? ctx.params.k : defaultTileSplitters<V, kBatch>(m_g, m_threads);
-        // Caller-owned outputs are idle until the merge writes them. The BWT buffer can hold the
-        // ranks only when the merge reads records from the lines (fused SA + BWT).
-        m_saScratch.reset(job.sa, job.sa ? static_cast<size_t>(job.totalLength) * sizeof(uint32_t) : 0);
-        m_bwtScratch.reset(job.sa && job.bwt && !job.rankOnly ? job.bwt : nullptr, job.bwt ? static_cast<size_t>(job.totalLength) : 0);
+        resetScratch();
     }
 
     ~Pipeline() {
@@ -622,6 +627,11 @@ class Pipeline {
         return SADCS_OK;
     }
 
+    // The same by prefix sort (cover 32's sample); done = false where run() is to be called instead.
+    int runPrefix(bool& done) {
+        return prefixBuild(done);
+    }
+
     const uint32_t* ranks() const {
         return m_ranks;
     }
@@ -644,6 +654,14 @@ class Pipeline {
     int m_threads = kMergeThreads;  // threads per merge tile
     ScratchStack m_saScratch;   // the caller's SA buffer before the merge
     ScratchStack m_bwtScratch;  // the caller's BWT buffer before the merge (fused builds)
+
+    // Caller-owned outputs are idle until the merge writes them. The BWT buffer can hold the
+    // ranks only when the merge reads records from the lines (fused SA + BWT).
+    void resetScratch() {
+        const Job& job = m_job;
+        m_saScratch.reset(job.sa, job.sa ? static_cast<size_t>(job.totalLength) * sizeof(uint32_t) : 0);
+        m_bwtScratch.reset(job.sa && job.bwt && !job.rankOnly ? job.bwt : nullptr, job.bwt ? static_cast<size_t>(job.totalLength) : 0);
+    }
 
     template <class T>
     int scratch(T*& pointer, uint64_t count) {
@@ -729,6 +747,35 @@ class Pipeline {
         return SADCS_OK;
     }
 
+    // The alphabet: dense codes 1..sigma for the bytes present, and their width (9 bits when all 256
+    // bytes occur: the code is then the byte plus one).
+    int alphabet(CodeTable& codes, int& sigma, int& charBits, uint32_t* byteCounts) {
+        if (!m_job.alphabetKnown) {
+            fillWords(byteCounts, 8, 0);
+            bytePresenceKernel<Texts><<<std::min<unsigned>(blocksFor((m_job.span + 15) / 16), 2048), 256, 0, m_stream>>>(
+                reinterpret_cast<const uint4*>(m_job.text), m_job.span, m_texts, byteCounts);
+            SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, byteCounts, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+            SADCS_HIP(hipStreamSynchronize(m_stream));
+            std::copy(m_ctx.hostWords, m_ctx.hostWords + 8, m_job.alphabetMask);
+            m_job.alphabetKnown = true;
+        }
+        codes = CodeTable{};
+        sigma = 0;
+        for (int b = 0; b < 256; b++) {
+            if ((m_job.alphabetMask[b / 32] >> (b % 32)) & 1u) {
+                codes.code[b] = static_cast<uint8_t>(++sigma);  // 256 wraps to 0 only if sigma = 256: see below
+            }
+        }
+        charBits = std::max(1, bitWidth(static_cast<uint64_t>(sigma)));
+        if (sigma == 256) {
+            // 9-bit codes do not fit a byte table; the key kernels use the byte plus one.
+            for (int b = 0; b < 256; b++) {
+                codes.code[b] = static_cast<uint8_t>(b);
+            }
+        }
+        return SADCS_OK;
+    }
+
     int rankSample() {
         const uint64_t rankWords = static_cast<uint64_t>(Cover::pack(m_job.span)) + CoverSet<V>::kSize + 8;
         if (!(V == kLinePositions && m_bwtScratch.take(m_ranks, rankWords))) {
@@ -793,28 +840,12 @@ class Pipeline {
             return status;
         }
 
-        // The alphabet: dense codes 1..sigma for the bytes present.
-        fillWords(byteCounts, 8, 0);
-        bytePresenceKernel<Texts><<<std::min<unsigned>(blocksFor((m_job.span + 15) / 16), 2048), 256, 0, m_stream>>>(
-            reinterpret_cast<const uint4*>(m_job.text), m_job.span, m_texts, byteCounts);
-        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords + 256, byteCounts, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
-        SADCS_HIP(hipStreamSynchronize(m_stream));
-        for (int b = 0; b < 256; b++) {
-            m_ctx.hostWords[b] = (m_ctx.hostWords[256 + b / 32] >> (b % 32)) & 1u;
-        }
         CodeTable codes{};
-        int sigma = 0;
-        for (int b = 0; b < 256; b++) {
-            if (m_ctx.hostWords[b]) {
-                codes.code[b] = static_cast<uint8_t>(++sigma);  // 256 wraps to 0 only if sigma = 256: see below
-            }
-        }
-        const int charBits = std::max(1, bitWidth(static_cast<uint64_t>(sigma)));
-        if (sigma == 256) {
-            // 9-bit codes do not fit a byte table; use the byte plus one computed in the key kernel.
-            for (int b = 0; b < 256; b++) {
-                codes.code[b] = static_cast<uint8_t>(b);
-            }
+        int sigma = 0, charBits = 0;
+        status = alphabet(codes, sigma, charBits, byteCounts);
+        if (status != SADCS_OK) {
+            cleanup();
+            return status;
         }
 
         RankParams rp{};
@@ -832,7 +863,7 @@ class Pipeline {
                 fillWords(textMasks, m_segments * 8, 0);
                 textPresenceKernel<<<static_cast<unsigned>((static_cast<uint64_t>(m_job.span) + 65535) / 65536), 256, 0, m_stream>>>(
                     reinterpret_cast<const uint4*>(m_job.text), m_job.span, m_texts, textMasks);
-                textCodesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(textMasks, m_segments, firstBits, textCodes, textShape);
+                textCodesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(textMasks, m_segments, firstBits, 64, textCodes, textShape);
                 SADCS_HIP(hipGetLastError());
                 rp.textCodes = textCodes;
                 rp.textShape = textShape;
@@ -840,6 +871,67 @@ class Pipeline {
         }
 
         initGroupIdsKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(m_job.deviceSegments, m_segments, groupIds[0]);
+
+        RankPassState state;
+        state.rp = rp;
+        state.codes = codes;
+        state.charBits = sigma == 256 ? 9 : charBits;
+        for (int i = 0; i < 2; i++) {
+            state.keys[i] = keys[i];
+            state.values[i] = values[i];
+            state.groupIds[i] = groupIds[i];
+        }
+        state.hist = hist;
+        state.sortAggregates = sortAggregates;
+        state.markAggregates = markAggregates;
+        state.counts = counts;
+        state.digits = digits;
+        state.u = M;
+        state.groups = m_segments;
+        state.first = true;
+        state.firstBits = firstBits;
+        status = rankPasses(state);
+        cleanup();
+        return status;
+    }
+
+    // The state of the ranking passes: the unresolved suffixes (u of them in `groups` groups that share
+    // `depth` characters; not listed before the first pass) and the buffers of a pass.
+    struct RankPassState {
+        RankParams rp{};
+        CodeTable codes{};
+        int charBits = 0;            // bits per character code; 9: all 256 bytes occur (code = byte + 1)
+        uint64_t* keys[2] = {};      // a list's ordinals are the words of keys[listBuffer]
+        uint32_t* values[2] = {};    // its compact indices values[listBuffer]
+        uint32_t* groupIds[2] = {};  // ordinal -> group id: groupIds[groupBuffer]
+        uint32_t* hist = nullptr;
+        Sum1* sortAggregates = nullptr;
+        MarkVec* markAggregates = nullptr;
+        uint32_t* counts = nullptr;
+        uint8_t* digits = nullptr;
+        uint32_t u = 0, groups = 0;
+        uint64_t depth = 0;
+        bool first = false;
+        int firstBits = 56;
+        int listBuffer = 1;
+        int groupBuffer = 0;
+    };
+
+    // Passes until every suffix has its rank.
+    int rankPasses(const RankPassState& state) {
+        const RankParams& rp = state.rp;
+        const CodeTable& codes = state.codes;
+        const int charBits = state.charBits;
+        const uint32_t M = rp.samples;
+        uint64_t* const* keys = state.keys;
+        uint32_t* const* values = state.values;
+        uint32_t* const* groupIds = state.groupIds;
+        uint32_t* hist = state.hist;
+        Sum1* sortAggregates = state.sortAggregates;
+        MarkVec* markAggregates = state.markAggregates;
+        uint32_t* counts = state.counts;
+        uint8_t* digits = state.digits;
+        const int firstBits = state.firstBits;
 
         SortBuffers<uint64_t> sb;
         sb.keys[0] = keys[0];
@@ -850,13 +942,13 @@ class Pipeline {
         sb.aggregates = sortAggregates;
         sb.digits = digits;
 
-        uint32_t u = M;
-        uint32_t groups = m_segments;
-        uint64_t depth = 0;
-        bool first = true;
-        int listBuffer = 1;  // where the list's t and ordinals are (values[x], keys[x] as words)
-        int gcur = 0;
-        const int rankBits = bitWidth(M);
+        uint32_t u = state.u;
+        uint32_t groups = state.groups;
+        uint64_t depth = state.depth;
+        bool first = state.first;
+        int listBuffer = state.listBuffer;  // where the list's t and ordinals are (values[x], keys[x] as words)
+        int gcur = state.groupBuffer;
+        const int rankBits = bitWidth(m_samples);
 
         while (u > 0) {
             if (!first && u <= kTailMax) {
@@ -864,7 +956,7 @@ class Pipeline {
                 TailParams tp{};
                 tp.rp = rp;
                 tp.codes = codes;
-                tp.charBits = sigma == 256 ? 9 : charBits;
+                tp.charBits = charBits;
                 tp.rankBits = rankBits;
                 tp.maxLength = m_job.maxLength;
                 tp.depth = depth;
@@ -885,8 +977,7 @@ class Pipeline {
                 times.doublingRounds += static_cast<int>(m_ctx.hostWords[1]);
                 if (m_ctx.hostWords[2] != 0) {
                     setError("sample ranking: groups left after doubling past the longest text (internal error)");
-                    cleanup();
-                    return SADCS_FAILED;
+                                        return SADCS_FAILED;
                 }
                 break;
             }
@@ -895,7 +986,7 @@ class Pipeline {
             if (depth < static_cast<uint64_t>(V)) {
                 spec.doubling = false;
                 spec.offset = static_cast<uint32_t>(depth);
-                spec.charBits = sigma == 256 ? 9 : charBits;
+                spec.charBits = charBits;
                 // The first pass sorts every sample: 56 key bits (7 digit passes) instead of up to 63
                 // (8) resolves nearly as many, and the later passes sort only the few left.
                 spec.chars = std::max(1, (first ? std::min(56, 64 - ordinalBits) : 64 - ordinalBits) / spec.charBits);
@@ -909,8 +1000,7 @@ class Pipeline {
                 const uint64_t h = depth / V * V;
                 if (h >= m_job.maxLength) {
                     setError("sample ranking: groups left at depth %llu (internal error)", static_cast<unsigned long long>(depth));
-                    cleanup();
-                    return SADCS_FAILED;
+                                        return SADCS_FAILED;
                 }
                 spec.doubling = true;
                 spec.offset = static_cast<uint32_t>(h);
@@ -923,7 +1013,7 @@ class Pipeline {
             const bool identity = first && !kBatch && u > 1;
             uint32_t* valuesOut = identity ? nullptr : values[y];
             uint8_t* digitsOut = first ? digits : nullptr;
-            if (sigma == 256 && !spec.doubling) {
+            if (charBits == 9 && !spec.doubling) {
                 makePassKeysKernel<V, Texts, true><<<blocksFor(u), 256, 0, m_stream>>>(
                     rp, m_texts, spec, codes, first, values[listBuffer], reinterpret_cast<const uint32_t*>(keys[listBuffer]), u, keys[y], valuesOut, digitsOut);
             } else {
@@ -968,7 +1058,7 @@ class Pipeline {
             ms.subkeyBits = spec.subkeyBits;
             ms.groupIds = groupIds[gcur];
             ms.ranks = m_ranks;
-            ms.sortedSample = m_lists[0];
+            ms.sortedSample = rp.sortedSample;
             ms.nextT = values[1 - c];
             ms.nextOrdinal = reinterpret_cast<uint32_t*>(keys[1 - c]);
             ms.nextGroupIds = groupIds[1 - gcur];
@@ -1003,7 +1093,647 @@ class Pipeline {
                 times.characterPasses++;
             }
         }
-        cleanup();
+        return SADCS_OK;
+    }
+
+    // ---- the prefix-sort path (prefix.h) ---------------------------------------------------------
+
+    // Device words read back by the host in one copy.
+    enum : uint32_t { kReadEqual = 0, kReadBigLeaves = 1, kReadBigRecords = 2, kReadLarge = 3, kReadWords = 8 };
+
+    // The whole build by prefix sort. done = false, with nothing allocated left, where the tile merge
+    // is the better path or the memory planned for this call does not hold this one.
+    int prefixBuild(bool& done) {
+        done = false;
+        auto since = std::chrono::steady_clock::now();
+        static_assert(V == 32, "the sample's ranks order ties within 32 characters");
+        const uint64_t N = m_job.totalLength;
+        CodeTable codes{};
+        int sigma = 0, charBits = 0;
+        uint32_t* byteCounts = nullptr;
+        SADCS_TRY(m_arena.allocate(byteCounts, 8));
+        const int alphabetStatus = alphabet(codes, sigma, charBits, byteCounts);
+        m_arena.release(byteCounts);
+        SADCS_TRY(alphabetStatus);
+        if (sigma == 256) {
+            charBits = 9;
+        }
+        const int segmentBits = m_segments > 1 ? bitWidth(m_segments - 1) : 0;
+        const int keyRoom = kPrefixKeyBits - segmentBits;
+        const int chars = std::min(kPrefixMaxChars, keyRoom / charBits);
+        // A tie group shares `chars` characters; large ones are merged as class lists, whose order
+        // within a group needs the characters up to the next sample position.
+        if (chars < kClasses - 1) {
+            return SADCS_OK;
+        }
+        const uint64_t budget = m_ctx.budget ? m_ctx.budget : m_ctx.arenaBytes;
+        // The caller's buffers hold results early on this path: nothing is borrowed from them.
+        m_saScratch.reset(nullptr, 0);
+        m_bwtScratch.reset(nullptr, 0);
+
+        struct Buffers {
+            uint32_t* sa = nullptr;
+            uint8_t* bwt = nullptr;
+            uint32_t *ties = nullptr, *words = nullptr, *firstRows = nullptr, *tableRows = nullptr;
+            uint64_t *startKeys = nullptr, *splitters = nullptr;
+            uint2* bigList = nullptr;
+            uint32_t* textMasks = nullptr;
+            uint8_t *textCodes = nullptr, *textShape = nullptr;
+        } b;
+        auto fits = [&](uint64_t bytes) { return m_arena.live() + bytes <= budget; };
+        auto take = [&](auto*& pointer, uint64_t count) {
+            using T = std::remove_reference_t<decltype(*pointer)>;
+            return fits(count * sizeof(T) + Arena::kAlign) && m_arena.tryAllocate(pointer, std::max<uint64_t>(count, 1));
+        };
+        auto releaseBase = [&]() {
+            m_arena.release(b.textShape);
+            m_arena.release(b.textCodes);
+            m_arena.release(b.textMasks);
+            m_arena.release(b.tableRows);
+            m_arena.release(b.splitters);
+            m_arena.release(b.bigList);
+            m_arena.release(b.startKeys);
+            m_arena.release(b.firstRows);
+            m_arena.release(b.words);
+            m_arena.release(b.ties);
+        };
+        auto giveUp = [&]() {
+            releaseBase();
+            m_arena.release(b.bwt);
+            m_arena.release(b.sa);
+            m_arena.release(m_ranks);
+            m_ctxMerge.ranks = nullptr;
+            resetScratch();
+            return SADCS_OK;
+        };
+
+        // Buckets and leaves.
+        const uint64_t leavesWanted = std::min<uint64_t>((N + kLeafTarget - 1) / kLeafTarget, static_cast<uint64_t>(kPrefixMaxBuckets) * kPrefixMaxBins);
+        uint32_t buckets = 1, bins = 1;
+        if (N > kLeafCapacity) {
+            buckets = static_cast<uint32_t>(leavesWanted);
+            if (leavesWanted > kPrefixMaxRoundBuckets) {
+                // Both levels about even: about 1.4 sqrt(leaves) buckets, a power of two.
+                buckets = 1;
+                while (buckets < kPrefixMaxBuckets && static_cast<uint64_t>(buckets) * buckets < 2 * leavesWanted) {
+                    buckets *= 2;
+                }
+                bins = static_cast<uint32_t>((leavesWanted + buckets - 1) / buckets);
+                if (bins > kPrefixMaxBins) {
+                    return giveUp();
+                }
+            }
+        }
+        const uint32_t leaves = buckets * bins;
+        const uint32_t tieWords = static_cast<uint32_t>((N + 31) / 32);
+        const uint32_t samples = buckets == 1 ? 0 : static_cast<uint32_t>(std::min<uint64_t>(N, static_cast<uint64_t>(leaves) * kOversample));
+
+        bool room = (m_job.sa || take(b.sa, m_job.span)) && (!m_job.wantBWT || m_job.bwt || take(b.bwt, m_job.span)) &&
+                    take(b.ties, tieWords + 4) && take(b.words, kReadWords) && take(b.startKeys, m_segments) && take(b.bigList, kBigLeavesMax) &&
+                    take(b.splitters, leaves) && take(b.tableRows, kPrefixMaxBuckets + 2) && (m_job.firstRows || take(b.firstRows, m_segments));
+        const bool ownCodes = kBatch && m_segments > 1 && sigma < 256;
+        if (ownCodes) {
+            room = room && take(b.textMasks, static_cast<uint64_t>(m_segments) * 8) && take(b.textCodes, static_cast<uint64_t>(m_segments) * 256) &&
+                   take(b.textShape, static_cast<uint64_t>(m_segments) * 2);
+        }
+        if (!room) {
+            return giveUp();
+        }
+
+        PrefixText pt{};
+        pt.words = reinterpret_cast<const uint64_t*>(m_job.text);
+        pt.span = m_job.span;
+        pt.segmentBits = segmentBits;
+        pt.charBits = charBits;
+        pt.chars = chars;
+        pt.wide = sigma == 256;
+        if constexpr (kBatch) {
+            if (ownCodes) {
+                fillWords(b.textMasks, static_cast<uint64_t>(m_segments) * 8, 0);
+                textPresenceKernel<<<static_cast<unsigned>((static_cast<uint64_t>(m_job.span) + 65535) / 65536), 256, 0, m_stream>>>(
+                    reinterpret_cast<const uint4*>(m_job.text), m_job.span, m_texts, b.textMasks);
+                textCodesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(b.textMasks, m_segments, keyRoom, kPrefixMaxChars, b.textCodes, b.textShape);
+                pt.textCodes = b.textCodes;
+                pt.textShape = b.textShape;
+            }
+        }
+        fillWords(b.words, kReadWords, 0);
+
+        RowOut out{};
+        out.sa = m_job.sa ? m_job.sa : b.sa;
+        out.bwt = m_job.wantBWT ? (m_job.bwt ? m_job.bwt : b.bwt) : nullptr;
+        out.ties = b.ties;
+        out.firstRows = m_job.firstRows ? m_job.firstRows : b.firstRows;
+        out.startKeys = b.startKeys;
+        out.segments = m_job.deviceSegments;
+        out.segmentBits = segmentBits;
+        auto mark = [&](double& phase, std::chrono::steady_clock::time_point& since) {
+            phase += secondsSince(since);
+            since = std::chrono::steady_clock::now();
+        };
+        bool sorted = false;
+        SADCS_TRY(prefixSort(pt, codes, out, b.splitters, b.tableRows, b.words, BigLeaves{b.words + kReadBigLeaves, b.bigList}, b.startKeys, tieWords, buckets, bins, samples, budget, sorted));
+        if (!sorted) {
+            return giveUp();
+        }
+        mark(times.classes, since);
+        bool ranked = false;
+        uint32_t tied = 0;
+        SADCS_TRY(prefixRank(codes, charBits, chars, out, tieWords, tied, budget, ranked));
+        if (!ranked) {
+            return giveUp();
+        }
+        mark(times.ranking, since);
+        bool ordered = true;
+        if (tied > 0) {
+            SADCS_TRY(orderTies(out, tieWords, tied, b.words + kReadLarge, budget, ordered));
+        }
+        if (!ordered) {
+            return giveUp();
+        }
+        if (kBatch && m_job.wantSA) {
+            localRowsKernel<Texts><<<std::min<unsigned>(blocksFor(N), 8192), 256, 0, m_stream>>>(m_texts, out.sa, static_cast<uint32_t>(N));
+            SADCS_HIP(hipGetLastError());
+        }
+        releaseBase();
+        m_arena.release(m_ranks);
+        m_ctxMerge.ranks = nullptr;
+        if (!m_job.wantSA) {
+            m_arena.release(b.sa);
+        }
+        m_outSA = b.sa;
+        m_outBWT = b.bwt;
+        m_ownBWT = b.bwt;
+        SADCS_TRY(sync());
+        mark(times.merge, since);
+        times.rankingBytes = times.classBytes = times.mergeBytes = m_arena.highWater();
+        if (m_timedMerge) {
+            float ms = 0;
+            SADCS_HIP(hipEventElapsedTime(&ms, m_ctx.kernelTimer[0], m_ctx.kernelTimer[1]));
+            times.mergeKernel = ms * 1e-3;
+        }
+        done = true;
+        return SADCS_OK;
+    }
+
+    // Steps 1 to 3 of prefix.h: every row of out.sa in key order, tie bits set, BWT bytes of rows that
+    // do not tie. sorted = false where the sample shows large groups throughout, or memory is short.
+    int prefixSort(const PrefixText& pt, const CodeTable& codes, const RowOut& out, uint64_t* splitters, uint32_t* tableRows, uint32_t* words, const BigLeaves& big,
+                   uint64_t* startKeys, uint32_t tieWords, uint32_t buckets, uint32_t bins, uint32_t samples, uint64_t budget, bool& sorted) {
+        sorted = false;
+        const uint64_t N = m_job.totalLength;
+        const uint32_t leaves = buckets * bins;
+        std::vector<void*> taken;
+        auto take = [&](auto*& pointer, uint64_t count) {
+            using T = std::remove_reference_t<decltype(*pointer)>;
+            if (m_arena.live() + count * sizeof(T) + Arena::kAlign > budget || !m_arena.tryAllocate(pointer, std::max<uint64_t>(count, 1))) {
+                return false;
+            }
+            taken.push_back(pointer);
+            return true;
+        };
+        auto releaseTaken = [&](size_t keep) {
+            while (taken.size() > keep) {
+                uint8_t* p = static_cast<uint8_t*>(taken.back());
+                m_arena.release(p);
+                taken.pop_back();
+            }
+        };
+
+        if (samples > 0) {
+            uint64_t* keys[2] = {};
+            uint32_t* values[2] = {};
+            uint32_t* hist = nullptr;
+            Sum1* aggregates = nullptr;
+            const bool small = samples <= kSampleCountMax;
+            bool room = take(keys[0], samples) && take(keys[1], samples) && take(values[0], samples);
+            if (!small) {
+                room = room && take(values[1], samples) && take(hist, radixHistWords(samples)) &&
+                       take(aggregates, radixAggregateBytes(samples) / sizeof(Sum1) + 1);
+            }
+            if (!room) {
+                releaseTaken(0);
+                return SADCS_OK;
+            }
+            samplePrefixesKernel<Texts><<<blocksFor(samples), 256, 0, m_stream>>>(pt, m_texts, codes, samples, keys[0], values[0]);
+            const uint64_t* sample = keys[1];
+            if (small) {
+                countSampleKernel<<<blocksFor(static_cast<uint64_t>((samples + kWave - 1) / kWave) * kSampleParts * kWave), 256, 0, m_stream>>>(keys[0], samples, values[0]);
+                placeSampleKernel<<<blocksFor(samples), 256, 0, m_stream>>>(keys[0], values[0], samples, keys[1]);
+            } else {
+                SortBuffers<uint64_t> sb;
+                for (int i = 0; i < 2; i++) {
+                    sb.keys[i] = keys[i];
+                    sb.values[i] = values[i];
+                }
+                sb.hist = hist;
+                sb.aggregates = aggregates;
+                sb.identityValues = true;
+                radixSort<uint64_t>(m_stream, sb, samples, 64 - kPrefixKeyBits, 64);
+                sample = sb.keys[sb.current];
+            }
+            pickSplittersKernel<<<std::min<unsigned>(blocksFor(std::max(samples, leaves)), 1024), 256, 0, m_stream>>>(sample, samples, leaves, splitters, words + kReadEqual);
+            SADCS_HIP(hipGetLastError());
+            releaseTaken(0);
+        }
+
+        // Bucket counts of the tiles, and from them the buckets' first rows.
+        const uint32_t blocks = static_cast<uint32_t>((static_cast<uint64_t>(m_job.span) + kPrefixBlock - 1) / kPrefixBlock);
+        const uint32_t tileBlocks = std::clamp<uint32_t>(blocks / 2048, 1, 16);
+        const uint32_t tiles = (blocks + tileBlocks - 1) / tileBlocks;
+        const int steps = log2Ceil(buckets);
+        uint32_t* offsets = nullptr;
+        Sum1* offsetAggregates = nullptr;
+        const uint64_t offsetWords = static_cast<uint64_t>(buckets) * tiles;
+        if (offsetWords > UINT32_MAX || !take(offsets, offsetWords) || !take(offsetAggregates, scanScratchBytes<Sum1, kSumItems>(offsetWords) / sizeof(Sum1) + 1)) {
+            releaseTaken(0);
+            return SADCS_OK;
+        }
+        countBucketsKernel<Texts><<<tiles, kPrefixThreads, 0, m_stream>>>(pt, m_texts, codes, splitters, buckets, bins, steps, tileBlocks, tiles, offsets);
+        exclusiveSum(m_stream, offsets, offsets, static_cast<uint32_t>(offsetWords), offsetAggregates);
+        bucketRowsKernel<<<blocksFor(buckets + 2), 256, 0, m_stream>>>(offsets, tiles, buckets, static_cast<uint32_t>(N), words + kReadEqual, tableRows);
+        SADCS_HIP(hipGetLastError());
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, tableRows, (buckets + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipStreamSynchronize(m_stream));
+        const std::vector<uint32_t> rows(m_ctx.hostWords, m_ctx.hostWords + buckets + 2);
+        // Sampled keys with 16 equal ones after them: their rows tie in groups of half a leaf or more.
+        if (static_cast<uint64_t>(rows[buckets + 1]) * kLargeTieShare > samples) {
+            releaseTaken(0);
+            return SADCS_OK;
+        }
+
+        fillWords(out.ties, tieWords + 4, 0);
+        if (out.bwt) {
+            startKeysKernel<Texts><<<blocksFor(m_segments), 256, 0, m_stream>>>(pt, m_texts, codes, m_job.deviceSegments, m_segments, startKeys);
+            firstBwtBytesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(m_job.text, m_job.deviceSegments, m_segments, out.bwt);
+        }
+
+        // The records a round holds: a key (and, two levels, a second key and a position) each, and
+        // the second level's counts.
+        const uint32_t maxRoundBuckets = std::min(buckets, kPrefixMaxRoundBuckets);
+        const uint64_t fixedBytes = 16 * Arena::kAlign + (2ull * maxRoundBuckets + 4 + static_cast<uint64_t>(maxRoundBuckets) * bins) * sizeof(uint32_t) +
+                                    (bins > 1 ? 2 * sizeof(uint32_t) * static_cast<uint64_t>(maxRoundBuckets) * bins : 0);
+        const uint64_t available = budget > m_arena.live() + fixedBytes ? budget - m_arena.live() - fixedBytes : 0;
+        // A large text's second level takes a quarter of a round at a time (fewer rounds, each of which
+        // reads the text again) in tiles of several blocks; a small one's launches would be too short.
+        const bool largeText = N >= (uint64_t(1) << 26);
+        const uint32_t tileRecords = largeText ? 4 * kPrefixBlock : kPrefixBlock;
+        const uint32_t binGroups = largeText ? 4 : 1;
+        const double perRecord = bins > 1 ? 12.0 + (8.0 + 2.0 * sizeof(uint32_t) * bins / tileRecords) / binGroups : 8.0;
+        const uint64_t capacity = std::min<uint64_t>(N, static_cast<uint64_t>(available / perRecord));
+        struct Round {
+            uint32_t first, count, rows;
+        };
+        // Runs of consecutive buckets of at most `most` rows and maxRoundBuckets buckets.
+        uint32_t largestBucket = 0;
+        for (uint32_t x = 0; x < buckets; x++) {
+            largestBucket = std::max(largestBucket, rows[x + 1] - rows[x]);
+        }
+        auto divide = [&](uint32_t first, uint32_t last, uint64_t most) {
+            std::vector<Round> runs;
+            for (uint32_t x = first; x < last;) {
+                Round r{x, 0, 0};
+                while (x < last && r.count < maxRoundBuckets && (r.count == 0 || static_cast<uint64_t>(r.rows) + (rows[x + 1] - rows[x]) <= most)) {
+                    r.rows += rows[x + 1] - rows[x];
+                    r.count++;
+                    x++;
+                }
+                runs.push_back(r);
+            }
+            return runs;
+        };
+        if (largestBucket > capacity) {
+            releaseTaken(0);
+            return SADCS_OK;  // one bucket is more than memory holds
+        }
+        const std::vector<Round> rounds = divide(0, buckets, capacity);
+        uint32_t largestRound = 0;
+        for (const Round& r : rounds) {
+            largestRound = std::max(largestRound, r.rows);
+        }
+        const uint32_t groupRows = bins > 1 ? std::max<uint32_t>(largestBucket, largestRound / binGroups) : largestRound;
+        uint64_t* keysA = nullptr;
+        uint64_t* keysB = nullptr;
+        uint32_t *positionsA = nullptr, *starts = nullptr, *tilesBefore = nullptr, *leafStart = nullptr, *binOffsets = nullptr;
+        Sum1* binAggregates = nullptr;
+        const uint64_t maxTiles = groupRows / tileRecords + maxRoundBuckets + 1;
+        bool room = take(keysA, largestRound) && take(starts, maxRoundBuckets + 1) && take(tilesBefore, maxRoundBuckets + 1) &&
+                    take(leafStart, static_cast<uint64_t>(maxRoundBuckets) * bins + 1);
+        if (bins > 1) {
+            room = room && take(keysB, groupRows) && take(positionsA, largestRound) && take(binOffsets, maxTiles * bins) &&
+                   take(binAggregates, scanScratchBytes<Sum1, kSumItems>(maxTiles * bins) / sizeof(Sum1) + 1);
+        }
+        if (!room || maxTiles * bins > UINT32_MAX) {
+            releaseTaken(0);
+            return SADCS_OK;
+        }
+
+        if (m_ctx.kernelTimer[0]) {
+            SADCS_HIP(hipEventRecord(m_ctx.kernelTimer[0], m_stream));
+        }
+        const size_t bucketShared = scatterSharedBytes<Texts>(), binShared = sizeof(PlaceStage);
+        SADCS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(scatterBucketsKernel<Texts>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bucketShared)));
+        SADCS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(scatterBinsKernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(binShared)));
+        for (const Round& r : rounds) {
+            if (r.rows == 0) {
+                continue;
+            }
+            const uint32_t rowBase = rows[r.first];
+            scatterBucketsKernel<Texts><<<tiles, kPrefixThreads, bucketShared, m_stream>>>(
+                pt, m_texts, codes, splitters, buckets, r.first, r.count, bins, log2Ceil(r.count), tileBlocks, tiles, offsets, rowBase, r.rows,
+                keysA, bins > 1 ? positionsA : out.sa + rowBase);
+            for (const Round& g : bins > 1 ? divide(r.first, r.first + r.count, groupRows) : std::vector<Round>{r}) {
+                if (g.rows == 0) {
+                    continue;
+                }
+                const uint32_t groupBase = rows[g.first];
+                bucketTilesKernel<<<1, kPrefixMaxRoundBuckets, 0, m_stream>>>(offsets, tiles, buckets, g.first, g.count, rowBase, static_cast<uint32_t>(N), tileRecords, starts, tilesBefore);
+                if (bins > 1) {
+                    const uint32_t groupTiles = g.rows / tileRecords + g.count + 1;
+                    const int binSteps = log2Ceil(bins);
+                    countBinsKernel<<<groupTiles, kPrefixThreads, 0, m_stream>>>(keysA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords, binOffsets);
+                    exclusiveSum(m_stream, binOffsets, binOffsets, groupTiles * bins, binAggregates);
+                    scatterBinsKernel<<<groupTiles, kPrefixThreads, binShared, m_stream>>>(keysA, positionsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords,
+                                                                                          binOffsets, g.rows, keysB, out.sa + groupBase);
+                }
+                leafStartsKernel<<<blocksFor(static_cast<uint64_t>(g.count) * bins + 1), 256, 0, m_stream>>>(starts, tilesBefore, binOffsets, g.count, bins, leafStart);
+                sortLeavesKernel<<<g.count * bins, kLeafThreads, 0, m_stream>>>(bins > 1 ? keysB : keysA, leafStart, groupBase, out, big);
+                SADCS_HIP(hipGetLastError());
+            }
+        }
+        if (m_ctx.kernelTimer[0]) {
+            SADCS_HIP(hipEventRecord(m_ctx.kernelTimer[1], m_stream));
+            m_timedMerge = true;
+            times.mergeElements = N;
+        }
+        releaseTaken(0);
+
+        // Leaves beyond a workgroup's LDS (equal keys, mostly), all at once by the radix sort.
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, big.count, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipStreamSynchronize(m_stream));
+        const uint32_t bigLeaves = m_ctx.hostWords[0], bigRecords = m_ctx.hostWords[1];
+        if (bigLeaves > 0) {
+            uint64_t* keys[2] = {};
+            uint32_t* values[2] = {};
+            uint32_t *hist = nullptr, *before = nullptr;
+            uint2* list = nullptr;
+            Sum1* aggregates = nullptr;
+            uint8_t* digits = nullptr;
+            bool bigRoom = bigLeaves <= kBigLeavesMax && take(before, bigLeaves + 1) && take(list, bigLeaves) && take(hist, radixHistWords(bigRecords)) &&
+                           take(aggregates, radixAggregateBytes(bigRecords) / sizeof(Sum1) + 1) && take(digits, bigRecords);
+            for (int i = 0; i < 2; i++) {
+                bigRoom = bigRoom && take(keys[i], bigRecords) && take(values[i], bigRecords);
+            }
+            if (!bigRoom) {
+                releaseTaken(0);
+                return SADCS_OK;
+            }
+            std::vector<uint2> leaf(bigLeaves);
+            SADCS_HIP(hipMemcpy(leaf.data(), big.list, bigLeaves * sizeof(uint2), hipMemcpyDeviceToHost));
+            std::sort(leaf.begin(), leaf.end(), [](const uint2& x, const uint2& y) { return x.x < y.x; });
+            std::vector<uint32_t> sums(bigLeaves + 1, 0);
+            for (uint32_t x = 0; x < bigLeaves; x++) {
+                sums[x + 1] = sums[x] + leaf[x].y;
+            }
+            SADCS_HIP(hipMemcpy(list, leaf.data(), bigLeaves * sizeof(uint2), hipMemcpyHostToDevice));
+            SADCS_HIP(hipMemcpy(before, sums.data(), (bigLeaves + 1) * sizeof(uint32_t), hipMemcpyHostToDevice));
+            bigLeafKeysKernel<Texts><<<blocksFor(bigRecords), 256, 0, m_stream>>>(pt, m_texts, codes, list, before, bigLeaves, bigRecords, out.sa, keys[0], values[0]);
+            SortBuffers<uint64_t> sb;
+            for (int i = 0; i < 2; i++) {
+                sb.keys[i] = keys[i];
+                sb.values[i] = values[i];
+            }
+            sb.hist = hist;
+            sb.aggregates = aggregates;
+            sb.digits = digits;
+            radixSort<uint64_t>(m_stream, sb, bigRecords, 64 - kPrefixKeyBits, 64);
+            bigLeafRowsKernel<<<blocksFor(bigRecords), 256, 0, m_stream>>>(sb.keys[sb.current], sb.values[sb.current], list, before, bigLeaves, bigRecords, out);
+            SADCS_HIP(hipGetLastError());
+            releaseTaken(0);
+        }
+        sorted = true;
+        return SADCS_OK;
+    }
+
+    // Step 4: the ranks of the sample suffixes (m_ranks). tied: rows that tie with a neighbour.
+    int prefixRank(const CodeTable& codes, int charBits, int chars, const RowOut& out, uint32_t tieWords, uint32_t& tied, uint64_t budget, bool& ranked) {
+        static_assert(V == 32, "the sample's ranks order ties within 32 characters");
+        ranked = false;
+        const uint32_t N = static_cast<uint32_t>(m_job.totalLength);
+        const uint32_t M = m_samples;
+        std::vector<void*> taken;
+        auto take = [&](auto*& pointer, uint64_t count) {
+            using T = std::remove_reference_t<decltype(*pointer)>;
+            if (m_arena.live() + count * sizeof(T) + Arena::kAlign > budget || !m_arena.tryAllocate(pointer, std::max<uint64_t>(count, 1))) {
+                return false;
+            }
+            taken.push_back(pointer);
+            return true;
+        };
+        auto drop = [&](auto*& pointer) {
+            for (size_t i = 0; i < taken.size(); i++) {
+                if (taken[i] == pointer) {
+                    taken.erase(taken.begin() + static_cast<std::ptrdiff_t>(i));
+                    break;
+                }
+            }
+            m_arena.release(pointer);
+        };
+        auto releaseTaken = [&]() {
+            while (!taken.empty()) {
+                uint8_t* p = static_cast<uint8_t*>(taken.back());
+                m_arena.release(p);
+                taken.pop_back();
+            }
+        };
+        const uint64_t rankWords = static_cast<uint64_t>(DifferenceCover<V>::pack(m_job.span)) + CoverSet<V>::kSize + 8;
+        uint32_t *index = nullptr, *group = nullptr, *counts = nullptr;
+        SampleVec* sampleAggregates = nullptr;
+        GroupVec* groupAggregates = nullptr;
+        Sum1* tieAggregates = nullptr;
+        const uint64_t tieBytes = scanScratchBytes<Sum1, kSumItems>(tieWords);
+        if (m_arena.live() + rankWords * sizeof(uint32_t) + Arena::kAlign > budget || !m_arena.tryAllocate(m_ranks, rankWords)) {
+            return SADCS_OK;
+        }
+        bool room = take(index, M) && take(group, M) && take(counts, 8) && take(sampleAggregates, scanScratchBytes<SampleVec, kSampleItems>(N) / sizeof(SampleVec) + 1) &&
+                    take(groupAggregates, scanScratchBytes<GroupVec, kMarkItems>(M) / sizeof(GroupVec) + 1) && take(tieAggregates, tieBytes / sizeof(Sum1) + 1);
+        if (!room) {
+            releaseTaken();
+            return SADCS_OK;
+        }
+        fillWords(m_ranks, rankWords, 0);
+        scanPipeline<SampleVec, kSampleItems>(m_stream, N, SampleProducer<V>{out.sa, out.ties}, SampleConsumer<V>{out.sa, index, group, M}, sampleAggregates);
+        const GroupProducer groups{group, M};
+        const uint32_t groupTiles = std::max<uint32_t>(1, ceilDiv(M, uint64_t(kScanThreads) * kMarkItems));
+        scanReduceKernel<GroupVec, kMarkItems><<<groupTiles, kScanThreads, 0, m_stream>>>(groups, M, groupAggregates);
+        scanAggregatesKernel<GroupVec><<<1, kScanThreads, 0, m_stream>>>(groupAggregates, groupTiles);
+        const uint32_t tieTiles = std::max<uint32_t>(1, ceilDiv(tieWords, uint64_t(kScanThreads) * kSumItems));
+        scanReduceKernel<Sum1, kSumItems><<<tieTiles, kScanThreads, 0, m_stream>>>(TieProducer{out.ties}, tieWords, tieAggregates);
+        scanAggregatesKernel<Sum1><<<1, kScanThreads, 0, m_stream>>>(tieAggregates, tieTiles);
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, groupAggregates + groupTiles, sizeof(GroupVec), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords + 4, tieAggregates + tieTiles, sizeof(Sum1), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipStreamSynchronize(m_stream));
+        const uint32_t unresolved = m_ctx.hostWords[1], unresolvedGroups = m_ctx.hostWords[2];
+        tied = m_ctx.hostWords[4];
+
+        RankPassState state;
+        if (unresolved > 0) {
+            room = take(state.keys[1], unresolved) && take(state.values[1], unresolved) && take(state.groupIds[0], unresolved / 2 + 2);
+            if (!room) {
+                releaseTaken();
+                return SADCS_OK;
+            }
+            scanDownsweepKernel<GroupVec, kMarkItems><<<groupTiles, kScanThreads, 0, m_stream>>>(
+                groups, GroupConsumer{index, m_ranks, state.values[1], reinterpret_cast<uint32_t*>(state.keys[1]), state.groupIds[0]}, M, groupAggregates);
+        }
+        const uint32_t rankCount = static_cast<uint32_t>(DifferenceCover<V>::pack(m_job.span));
+        const uint64_t windows = std::max<uint64_t>(1, (uint64_t(rankCount) * sizeof(uint32_t) + kDeferredRankWindow - 1) / kDeferredRankWindow);
+        const uint32_t step = static_cast<uint32_t>((rankCount + windows - 1) / windows);
+        for (uint32_t lo = 0; lo < rankCount; lo += step) {
+            scatterSortedRanksKernel<<<std::min<unsigned>(blocksFor(M), 8192), 256, 0, m_stream>>>(index, M, lo, std::min(rankCount, lo + step), m_ranks);
+        }
+        SADCS_HIP(hipGetLastError());
+        m_ctxMerge.ranks = m_ranks;
+        if (unresolved > 0) {
+            // Stream order keeps the kernels above ahead of any reuse of these buffers.
+            drop(index);
+            drop(group);
+            room = take(state.keys[0], unresolved) && take(state.values[0], unresolved) && take(state.groupIds[1], unresolved / 2 + 2) &&
+                   take(state.hist, radixHistWords(unresolved)) && take(state.sortAggregates, radixAggregateBytes(unresolved) / sizeof(Sum1) + 1) &&
+                   take(state.markAggregates, scanScratchBytes<MarkVec, kMarkItems>(unresolved) / sizeof(MarkVec) + 1) && take(state.digits, unresolved);
+            if (!room) {
+                releaseTaken();
+                return SADCS_OK;
+            }
+            state.rp.text = reinterpret_cast<const uint64_t*>(m_job.text);
+            state.rp.ranks = m_ranks;
+            state.rp.samples = 0;  // no list of the sorted sample is kept
+            state.rp.segments = m_segments;
+            state.rp.segmentTable = m_job.deviceSegments;
+            state.codes = codes;
+            state.charBits = charBits;
+            state.counts = counts;
+            state.u = unresolved;
+            state.groups = unresolvedGroups;
+            state.depth = static_cast<uint64_t>(chars);
+            times.characterPasses++;
+            const int status = rankPasses(state);
+            if (status != SADCS_OK) {
+                releaseTaken();
+                return status;
+            }
+        }
+        releaseTaken();
+        ranked = true;
+        return SADCS_OK;
+    }
+
+    // Step 5: the rows that tie, in order.
+    int orderTies(const RowOut& out, uint32_t tieWords, uint32_t tied, uint32_t* largeCount, uint64_t budget, bool& ordered) {
+        static_assert(V == 32, "the sample's ranks order ties within 32 characters");
+        ordered = false;
+        std::vector<void*> taken;
+        auto take = [&](auto*& pointer, uint64_t count) {
+            using T = std::remove_reference_t<decltype(*pointer)>;
+            if (m_arena.live() + count * sizeof(T) + Arena::kAlign > budget || !m_arena.tryAllocate(pointer, std::max<uint64_t>(count, 1))) {
+                return false;
+            }
+            taken.push_back(pointer);
+            return true;
+        };
+        auto releaseTaken = [&]() {
+            while (!taken.empty()) {
+                uint8_t* p = static_cast<uint8_t*>(taken.back());
+                m_arena.release(p);
+                taken.pop_back();
+            }
+        };
+        uint32_t* rows = nullptr;
+        uint8_t* flags = nullptr;
+        Sum1* aggregates = nullptr;
+        if (!take(rows, tied) || !take(flags, tied) || !take(aggregates, scanScratchBytes<Sum1, kSumItems>(tieWords) / sizeof(Sum1) + 1)) {
+            releaseTaken();
+            return SADCS_OK;
+        }
+        scanPipeline<Sum1, kSumItems>(m_stream, tieWords, TieProducer{out.ties}, TieConsumer{out.ties, rows}, aggregates);
+        const size_t shared = static_cast<size_t>(kTieRecords) * LdsRecords<V, kBatch>::bytesPerRecord();
+        tieGroupsKernel<Texts><<<blocksFor(tied, kTieTile), kTieTile, shared, m_stream>>>(m_ctxMerge, m_texts, rows, tied, out, flags, largeCount);
+        SADCS_HIP(hipGetLastError());
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, largeCount, sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipStreamSynchronize(m_stream));
+        const uint32_t large = m_ctx.hostWords[0];
+        if (large > 0) {
+            // Class lists of the large groups, each in suffix order, merged like a text's own.
+            uint32_t *largeRow = nullptr, *order = nullptr, *classStart = nullptr, *hist = nullptr, *errors = nullptr;
+            uint64_t* keys[2] = {};
+            uint32_t* values[2] = {};
+            uint8_t* digits = nullptr;
+            Sum1* sortAggregates = nullptr;
+            LargeVec* largeAggregates = nullptr;
+            bool room = take(largeRow, large) && take(order, large) && take(classStart, kMaxLists + 1) && take(errors, 2) && take(hist, radixHistWords(large)) &&
+                        take(sortAggregates, radixAggregateBytes(large) / sizeof(Sum1) + 1) && take(digits, large) &&
+                        take(largeAggregates, scanScratchBytes<LargeVec, kLargeItems>(tied) / sizeof(LargeVec) + 1);
+            for (int i = 0; i < 2; i++) {
+                room = room && take(keys[i], large) && take(values[i], large);
+            }
+            // The merge's own levels: splitters, rows and counts of about half a word per element.
+            if (!room || m_arena.live() + static_cast<uint64_t>(large) + (1u << 20) > budget) {
+                releaseTaken();
+                return SADCS_OK;
+            }
+                        const int rankBits = bitWidth(m_samples);
+            const int groupBits = bitWidth(large / kTieGroupMax);
+            const int classBits = bitWidth(kClasses);
+            fillWords(errors, 1, 0);
+            scanPipeline<LargeVec, kLargeItems>(m_stream, tied, LargeProducer{flags, rows},
+                                                LargeConsumer<V, Texts>{rows, out.sa, m_ranks, m_texts, m_job.span, groupBits, rankBits, largeRow, keys[0], values[0]}, largeAggregates);
+            SortBuffers<uint64_t> sb;
+            for (int i = 0; i < 2; i++) {
+                sb.keys[i] = keys[i];
+                sb.values[i] = values[i];
+            }
+            sb.hist = hist;
+            sb.aggregates = sortAggregates;
+            sb.digits = digits;
+            radixSort<uint64_t>(m_stream, sb, large, 0, rankBits + groupBits + classBits);
+            classStartsKernel<<<1, kWave, 0, m_stream>>>(sb.keys[sb.current], large, rankBits + groupBits, kClasses, classStart);
+            SADCS_HIP(hipGetLastError());
+            SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, classStart, (kClasses + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+            SADCS_HIP(hipStreamSynchronize(m_stream));
+            const uint32_t* positions = sb.values[sb.current];
+            ListSet lists{};
+            lists.count = kClasses;
+            for (int d = 0; d < kClasses; d++) {
+                lists.ptr[d] = positions + m_ctx.hostWords[d];
+                lists.length[d] = m_ctx.hostWords[d + 1] - m_ctx.hostWords[d];
+                lists.indexBase[d] = m_ctx.hostWords[d];
+            }
+            lists.indexBase[kClasses] = m_ctx.hostWords[kClasses];
+            TileOut tileOut{};
+            tileOut.index = order;
+            const int status = mergeLevel<kOutIndex>(lists, tileOut, errors);
+            if (status == SADCS_NOT_ENOUGH_MEMORY) {
+                releaseTaken();
+                return SADCS_OK;
+            }
+            if (status != SADCS_OK) {
+                releaseTaken();
+                return status;
+            }
+            largeRowsKernel<Texts><<<blocksFor(large), 256, 0, m_stream>>>(m_ctxMerge, m_texts, largeRow, positions, order, large, out);
+            if (out.bwt) {
+                largeBytesKernel<Texts><<<blocksFor(large), 256, 0, m_stream>>>(m_ctxMerge, m_texts, largeRow, large, out);
+            }
+            SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, errors, sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+            SADCS_HIP(hipStreamSynchronize(m_stream));
+            if (m_ctx.hostWords[0] != 0) {
+                setError("tie groups: inconsistent tile layout (internal error, code %u)", m_ctx.hostWords[0]);
+                releaseTaken();
+                return SADCS_FAILED;
+            }
+        }
+        releaseTaken();
+        ordered = true;
         return SADCS_OK;
     }
 
@@ -2169,7 +2899,25 @@ int buildWith(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, Text
     uint32_t* outSA = nullptr;
     uint8_t* outBWT = nullptr;
     std::unique_ptr<Pipeline<V, Texts>> keep;
-    const int status = runPipeline<V, Texts>(ctx, job, texts, times, &outSA, &outBWT, keep);
+    std::unique_ptr<Pipeline<32, Texts>> prefix;
+    int status = SADCS_OK;
+    bool done = false;
+    // The prefix sort, whatever the cover (it compares the few suffixes left by cover 32's sample),
+    // unless merge parameters ask for the tile merge.
+    if (!job.rankOnly && !ctx.params.tiles) {
+        prefix.reset(new Pipeline<32, Texts>(ctx, job, texts));
+        status = prefix->runPrefix(done);
+        if (done) {
+            times = prefix->times;
+            outSA = prefix->m_outSA;
+            outBWT = prefix->m_outBWT;
+        } else {
+            prefix.reset();
+        }
+    }
+    if (status == SADCS_OK && !done) {
+        status = runPipeline<V, Texts>(ctx, job, texts, times, &outSA, &outBWT, keep);
+    }
     size_t deviceBytes = arena.highWater();
     if (deviceCall) {
         deviceBytes += static_cast<size_t>(layout.span) + kTextPadding;
@@ -2408,7 +3156,12 @@ int buildOn(sadcs_ctx* context, const Params& params, const Layout& layout, cons
             setError("input needs %zu bytes of the context's %zu", need, context->arenaBytes);
             return SADCS_NOT_ENOUGH_MEMORY;
         }
-        return build(*context, layout, rq, stats);
+        // A device call keeps to its own plan (10 bytes per input byte with the caller's buffers)
+        // on a context planned for host calls, unless the difference is small.
+        context->budget = deviceCall ? std::max(need, std::min(context->arenaBytes, kFreeBudget)) : 0;
+        const int status = build(*context, layout, rq, stats);
+        context->budget = 0;
+        return status;
     }
     const auto start = std::chrono::steady_clock::now();
     sadcs_ctx planner;

@@ -247,8 +247,55 @@ struct StoreExclusiveU32 {
 
 constexpr int kSumItems = 16;
 
-// Exclusive sum of count words, in place allowed.
+// Exclusive sum of up to kOneBlockSum words in one workgroup, 16 words a thread at a time.
+constexpr uint32_t kOneBlockSum = 32768;
+constexpr int kOneBlockThreads = 1024;
+
+__global__ __launch_bounds__(kOneBlockThreads) void exclusiveSumKernel(const uint32_t* in, uint32_t* out, uint32_t count) {
+    __shared__ uint32_t waveTotals[kOneBlockThreads / kWave];
+    const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    uint32_t carry = 0;
+    for (uint32_t chunk = 0; chunk < count; chunk += kOneBlockThreads * kSumItems) {
+        // A wave's 64 * 16 words lane after lane: striped loads, a scan per 64.
+        const uint32_t base = chunk + wave * kWave * kSumItems + lane;
+        uint32_t x[kSumItems], before[kSumItems];
+#pragma unroll
+        for (int j = 0; j < kSumItems; j++) {
+            x[j] = base + j * kWave < count ? in[base + j * kWave] : 0;
+        }
+        uint32_t total = 0;
+#pragma unroll
+        for (int j = 0; j < kSumItems; j++) {
+            const uint32_t inclusive = waveInclusive<OpSum>(x[j]);
+            before[j] = total + inclusive - x[j];
+            total += readLane(inclusive, kWave - 1);
+        }
+        if (lane == 0) {
+            waveTotals[wave] = total;
+        }
+        __syncthreads();
+        uint32_t prefix = carry;
+        for (uint32_t w = 0; w < kOneBlockThreads / kWave; w++) {
+            prefix += w < wave ? waveTotals[w] : 0;
+            carry += waveTotals[w];
+        }
+#pragma unroll
+        for (int j = 0; j < kSumItems; j++) {
+            if (base + j * kWave < count) {
+                out[base + j * kWave] = prefix + before[j];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Exclusive sum of count words, in place allowed. Few words take one launch instead of three: the
+// passes over a few hundred thousand keys, whose tile histograms these are, are bound by launches.
 inline void exclusiveSum(hipStream_t stream, const uint32_t* in, uint32_t* out, uint32_t count, Sum1* aggregates) {
+    if (count <= kOneBlockSum) {
+        exclusiveSumKernel<<<1, kOneBlockThreads, 0, stream>>>(in, out, count);
+        return;
+    }
     scanPipeline<Sum1, kSumItems>(stream, count, LoadU32{in}, StoreExclusiveU32{out}, aggregates);
 }
 

@@ -251,8 +251,8 @@ __global__ __launch_bounds__(256) void textPresenceKernel(const uint4* __restric
 }
 
 // Per text: codes 1..sigma of its bytes in byte order (0 for absent bytes; sigma < 256), the code
-// width and the characters that fit subkeyBits.
-__global__ void textCodesKernel(const uint32_t* __restrict__ textMasks, uint32_t texts, int subkeyBits, uint8_t* __restrict__ textCodes, uint8_t* __restrict__ textShape) {
+// width and the characters that fit subkeyBits (at most maxChars).
+__global__ void textCodesKernel(const uint32_t* __restrict__ textMasks, uint32_t texts, int subkeyBits, int maxChars, uint8_t* __restrict__ textCodes, uint8_t* __restrict__ textShape) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= texts) {
         return;
@@ -265,7 +265,7 @@ __global__ void textCodesKernel(const uint32_t* __restrict__ textMasks, uint32_t
     }
     const int bits = count > 1 ? 32 - __clz(count) : 1;
     textShape[2 * s] = static_cast<uint8_t>(bits);
-    textShape[2 * s + 1] = static_cast<uint8_t>(max(1, subkeyBits / bits));
+    textShape[2 * s + 1] = static_cast<uint8_t>(min(maxChars, max(1, subkeyBits / bits)));
 }
 
 // The sort of a pass after the first, when its groups are small. The list arrives grouped: keys
