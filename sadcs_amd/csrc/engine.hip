@@ -1168,7 +1168,10 @@ class Pipeline {
         };
 
         // Buckets and leaves.
-        const uint64_t leavesWanted = std::min<uint64_t>((N + kLeafTarget - 1) / kLeafTarget, static_cast<uint64_t>(kPrefixMaxBuckets) * kPrefixMaxBins);
+        // Few leaves: larger ones from a smaller sample, which sorts by counting.
+        const bool coarse = N <= static_cast<uint64_t>(kSampleCountMax) * kCoarseLeaf / kCoarseOversample;
+        const uint32_t leafTarget = coarse ? kCoarseLeaf : kLeafTarget;
+        const uint64_t leavesWanted = std::min<uint64_t>((N + leafTarget - 1) / leafTarget, static_cast<uint64_t>(kPrefixMaxBuckets) * kPrefixMaxBins);
         uint32_t buckets = 1, bins = 1;
         if (N > kLeafCapacity) {
             buckets = static_cast<uint32_t>(leavesWanted);
@@ -1186,7 +1189,7 @@ class Pipeline {
         }
         const uint32_t leaves = buckets * bins;
         const uint32_t tieWords = static_cast<uint32_t>((N + 31) / 32);
-        const uint32_t samples = buckets == 1 ? 0 : static_cast<uint32_t>(std::min<uint64_t>(N, static_cast<uint64_t>(leaves) * kOversample));
+        const uint32_t samples = buckets == 1 ? 0 : static_cast<uint32_t>(std::min<uint64_t>(N, static_cast<uint64_t>(leaves) * (coarse ? kCoarseOversample : kOversample)));
 
         bool room = (m_job.sa || take(b.sa, m_job.span)) && (!m_job.wantBWT || m_job.bwt || take(b.bwt, m_job.span)) &&
                     take(b.ties, tieWords + 4) && take(b.words, kReadWords) && take(b.startKeys, m_segments) && take(b.bigList, kBigLeavesMax) &&
@@ -1246,13 +1249,13 @@ class Pipeline {
         mark(times.ranking, since);
         bool ordered = true;
         if (tied > 0) {
-            SADCS_TRY(orderTies(out, tieWords, tied, b.words + kReadLarge, budget, ordered));
+            SADCS_TRY(orderTies(out, chars, tieWords, tied, b.words + kReadLarge, budget, ordered));
         }
         if (!ordered) {
             return giveUp();
         }
         if (kBatch && m_job.wantSA) {
-            localRowsKernel<Texts><<<std::min<unsigned>(blocksFor(N), 8192), 256, 0, m_stream>>>(m_texts, out.sa, static_cast<uint32_t>(N));
+            localRowsKernel<<<blocksFor(N, 256 * kLocalItems), 256, 0, m_stream>>>(m_job.deviceSegments, m_segments, out.sa, static_cast<uint32_t>(N));
             SADCS_HIP(hipGetLastError());
         }
         releaseBase();
@@ -1368,8 +1371,7 @@ class Pipeline {
             firstBwtBytesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(m_job.text, m_job.deviceSegments, m_segments, out.bwt);
         }
 
-        // The records a round holds: a key (and, two levels, a second key and a position) each, and
-        // the second level's counts.
+        // The records a round holds and, two levels, a group of its buckets' records again and counts.
         const uint32_t maxRoundBuckets = std::min(buckets, kPrefixMaxRoundBuckets);
         const uint64_t fixedBytes = 16 * Arena::kAlign + (2ull * maxRoundBuckets + 4 + static_cast<uint64_t>(maxRoundBuckets) * bins) * sizeof(uint32_t) +
                                     (bins > 1 ? 2 * sizeof(uint32_t) * static_cast<uint64_t>(maxRoundBuckets) * bins : 0);
@@ -1378,8 +1380,8 @@ class Pipeline {
         // reads the text again) in tiles of several blocks; a small one's launches would be too short.
         const bool largeText = N >= (uint64_t(1) << 26);
         const uint32_t tileRecords = largeText ? 4 * kPrefixBlock : kPrefixBlock;
-        const uint32_t binGroups = largeText ? 4 : 1;
-        const double perRecord = bins > 1 ? 12.0 + (8.0 + 2.0 * sizeof(uint32_t) * bins / tileRecords) / binGroups : 8.0;
+        const uint32_t binGroups = N >= (uint64_t(1) << 29) ? 8 : largeText ? 4 : 1;
+        const double perRecord = sizeof(PrefixRecord) * 1.0 + (bins > 1 ? (sizeof(PrefixRecord) + 2.0 * sizeof(uint32_t) * bins / tileRecords) / binGroups : 0.0);
         const uint64_t capacity = std::min<uint64_t>(N, static_cast<uint64_t>(available / perRecord));
         struct Round {
             uint32_t first, count, rows;
@@ -1412,15 +1414,14 @@ class Pipeline {
             largestRound = std::max(largestRound, r.rows);
         }
         const uint32_t groupRows = bins > 1 ? std::max<uint32_t>(largestBucket, largestRound / binGroups) : largestRound;
-        uint64_t* keysA = nullptr;
-        uint64_t* keysB = nullptr;
-        uint32_t *positionsA = nullptr, *starts = nullptr, *tilesBefore = nullptr, *leafStart = nullptr, *binOffsets = nullptr;
+        PrefixRecord *recordsA = nullptr, *recordsB = nullptr;
+        uint32_t *starts = nullptr, *tilesBefore = nullptr, *leafStart = nullptr, *binOffsets = nullptr;
         Sum1* binAggregates = nullptr;
         const uint64_t maxTiles = groupRows / tileRecords + maxRoundBuckets + 1;
-        bool room = take(keysA, largestRound) && take(starts, maxRoundBuckets + 1) && take(tilesBefore, maxRoundBuckets + 1) &&
+        bool room = take(recordsA, largestRound) && take(starts, maxRoundBuckets + 1) && take(tilesBefore, maxRoundBuckets + 1) &&
                     take(leafStart, static_cast<uint64_t>(maxRoundBuckets) * bins + 1);
         if (bins > 1) {
-            room = room && take(keysB, groupRows) && take(positionsA, largestRound) && take(binOffsets, maxTiles * bins) &&
+            room = room && take(recordsB, groupRows) && take(binOffsets, maxTiles * bins) &&
                    take(binAggregates, scanScratchBytes<Sum1, kSumItems>(maxTiles * bins) / sizeof(Sum1) + 1);
         }
         if (!room || maxTiles * bins > UINT32_MAX) {
@@ -1440,8 +1441,7 @@ class Pipeline {
             }
             const uint32_t rowBase = rows[r.first];
             scatterBucketsKernel<Texts><<<tiles, kPrefixThreads, bucketShared, m_stream>>>(
-                pt, m_texts, codes, splitters, buckets, r.first, r.count, bins, log2Ceil(r.count), tileBlocks, tiles, offsets, rowBase, r.rows,
-                keysA, bins > 1 ? positionsA : out.sa + rowBase);
+                pt, m_texts, codes, splitters, buckets, r.first, r.count, bins, log2Ceil(r.count), tileBlocks, tiles, offsets, rowBase, r.rows, recordsA);
             for (const Round& g : bins > 1 ? divide(r.first, r.first + r.count, groupRows) : std::vector<Round>{r}) {
                 if (g.rows == 0) {
                     continue;
@@ -1451,13 +1451,14 @@ class Pipeline {
                 if (bins > 1) {
                     const uint32_t groupTiles = g.rows / tileRecords + g.count + 1;
                     const int binSteps = log2Ceil(bins);
-                    countBinsKernel<<<groupTiles, kPrefixThreads, 0, m_stream>>>(keysA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords, binOffsets);
+                    countBinsKernel<<<groupTiles, kPrefixThreads, 0, m_stream>>>(recordsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords, binOffsets);
                     exclusiveSum(m_stream, binOffsets, binOffsets, groupTiles * bins, binAggregates);
-                    scatterBinsKernel<<<groupTiles, kPrefixThreads, binShared, m_stream>>>(keysA, positionsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords,
-                                                                                          binOffsets, g.rows, keysB, out.sa + groupBase);
+                    scatterBinsKernel<<<groupTiles, kPrefixThreads, binShared, m_stream>>>(recordsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords,
+                                                                                          binOffsets, g.rows, recordsB);
                 }
                 leafStartsKernel<<<blocksFor(static_cast<uint64_t>(g.count) * bins + 1), 256, 0, m_stream>>>(starts, tilesBefore, binOffsets, g.count, bins, leafStart);
-                sortLeavesKernel<<<g.count * bins, kLeafThreads, 0, m_stream>>>(bins > 1 ? keysB : keysA, leafStart, groupBase, out, big);
+                const auto sortLeaves = N > static_cast<uint64_t>(leaves) * kLeafTarget ? sortLeavesKernel<2 * kLeafCapacity> : sortLeavesKernel<kLeafCapacity>;
+                sortLeaves<<<g.count * bins, kLeafThreads, 0, m_stream>>>(bins > 1 ? recordsB : recordsA, leafStart, groupBase, out, big);
                 SADCS_HIP(hipGetLastError());
             }
         }
@@ -1629,7 +1630,7 @@ class Pipeline {
     }
 
     // Step 5: the rows that tie, in order.
-    int orderTies(const RowOut& out, uint32_t tieWords, uint32_t tied, uint32_t* largeCount, uint64_t budget, bool& ordered) {
+    int orderTies(const RowOut& out, int chars, uint32_t tieWords, uint32_t tied, uint32_t* largeCount, uint64_t budget, bool& ordered) {
         static_assert(V == 32, "the sample's ranks order ties within 32 characters");
         ordered = false;
         std::vector<void*> taken;
@@ -1656,8 +1657,7 @@ class Pipeline {
             return SADCS_OK;
         }
         scanPipeline<Sum1, kSumItems>(m_stream, tieWords, TieProducer{out.ties}, TieConsumer{out.ties, rows}, aggregates);
-        const size_t shared = static_cast<size_t>(kTieRecords) * LdsRecords<V, kBatch>::bytesPerRecord();
-        tieGroupsKernel<Texts><<<blocksFor(tied, kTieTile), kTieTile, shared, m_stream>>>(m_ctxMerge, m_texts, rows, tied, out, flags, largeCount);
+        tieGroupsKernel<Texts><<<blocksFor(tied, kTieTile), kTieTile, 0, m_stream>>>(m_ctxMerge, m_texts, static_cast<uint32_t>(chars), rows, tied, out, flags, largeCount);
         SADCS_HIP(hipGetLastError());
         SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, largeCount, sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
         SADCS_HIP(hipStreamSynchronize(m_stream));

@@ -44,16 +44,36 @@ constexpr int kPrefixMaxChars = 24;      // characters of a key (one thread's wi
 constexpr uint32_t kPrefixMaxBuckets = 2048;       // first-level buckets
 constexpr uint32_t kPrefixMaxRoundBuckets = 512;   // of them in one round (their tables share the LDS with the records)
 constexpr uint32_t kPrefixMaxBins = 512;           // leaves of a bucket
-constexpr uint32_t kLeafCapacity = 4096;           // records a leaf's workgroup sorts in LDS
-// Records of a leaf on average and sampled keys per leaf: a leaf's size then spreads by a quarter
-// around 1536, and one of more than 4096 without equal keys is about one in a million.
-constexpr uint32_t kLeafTarget = 1536;
-constexpr uint32_t kOversample = 16;
+// Records of a leaf on average, the most its workgroup sorts in LDS, and sampled keys per leaf: a
+// leaf's size spreads by a sixth around its average, and one of twice that without equal keys is
+// about one in 200,000. Leaves of 1024 in 27 KB, five workgroups a CU, sort 1 GiB in 12.3 ms;
+// 1536 in 40 KB 14.2, 1536 in 53 KB 18.4. Beyond 2^30 rows the most leaves there are hold up to 2048.
+constexpr uint32_t kLeafTarget = 1024;
+constexpr uint32_t kLeafCapacity = 2048;
+constexpr uint32_t kOversample = 32;
+// Up to about 2.3 million rows: leaves of 1536 on average, of up to 4096, from 16 keys a leaf.
+constexpr uint32_t kCoarseLeaf = 1536;
+constexpr uint32_t kCoarseOversample = 16;
 constexpr uint32_t kTieGroupMax = 24;              // rows of a group compared in LDS
 constexpr uint64_t kLargeTieShare = 16;            // at most 1 / this of the sample in large groups
 
-__device__ __forceinline__ uint64_t keyPart(uint64_t record) {
-    return record & ~uint64_t(0xFF);
+// A suffix on its way to its row: its key (the character before it in the low byte) and position, 12
+// bytes together, so that a run of records is one run of memory: keys and positions apart wrote a
+// third more lines.
+struct PrefixRecord {
+    uint32_t low, high, position;
+};
+
+__device__ __forceinline__ PrefixRecord packRecord(uint64_t key, uint32_t position) {
+    return PrefixRecord{static_cast<uint32_t>(key), static_cast<uint32_t>(key >> 32), position};
+}
+
+__device__ __forceinline__ uint64_t keyOf(const PrefixRecord& r) {
+    return static_cast<uint64_t>(r.high) << 32 | r.low;
+}
+
+__device__ __forceinline__ uint64_t keyPart(uint64_t key) {
+    return key & ~uint64_t(0xFF);
 }
 
 // How a position's key is built: the text's index (a batch), then `chars` codes of `charBits` bits
@@ -172,7 +192,7 @@ __global__ __launch_bounds__(256) void placeSampleKernel(const uint64_t* __restr
 }
 
 // splitters[x] (x in [0, leaves - 1)) = the sorted sample's key at (x + 1) / leaves of its valid
-// part; equal[0] counts sampled keys equal to the one kOversample places on: a group of that key
+// part; equal[0] counts sampled keys equal to the one kCoarseOversample places on: a group of that key
 // holds about a leaf of rows or more.
 __global__ __launch_bounds__(256) void pickSplittersKernel(const uint64_t* __restrict__ sorted, uint32_t count, uint32_t leaves, uint64_t* __restrict__ splitters, uint32_t* __restrict__ equal) {
     uint32_t lo = 0, hi = count;  // the valid keys come before the ~0 ones
@@ -189,7 +209,7 @@ __global__ __launch_bounds__(256) void pickSplittersKernel(const uint64_t* __res
         if (x + 1 < leaves) {
             splitters[x] = lo > 0 ? sorted[static_cast<uint64_t>(lo) * (x + 1) / leaves] : ~uint64_t(0);
         }
-        ties += x + kOversample < lo && sorted[x] == sorted[x + kOversample] ? 1 : 0;
+        ties += x + kCoarseOversample < lo && sorted[x] == sorted[x + kCoarseOversample] ? 1 : 0;
     }
     for (int offset = kWave / 2; offset > 0; offset /= 2) {
         ties += __shfl_xor(ties, offset);
@@ -459,7 +479,7 @@ struct PlaceStage {
 // order so that each bin's records are written in a run; thread t holds bin t's next output index in
 // `cursor`. Order within a bin is not kept. The stage's records are read until the caller's next
 // barrier (placeBlock's own first one will do).
-__device__ __forceinline__ void placeBlock(PlaceStage& s, const uint64_t (&key)[kPrefixItems], const uint32_t (&position)[kPrefixItems], uint32_t valid, uint32_t bins, int steps, uint32_t& cursor, uint64_t* __restrict__ keysOut, uint32_t* __restrict__ positionsOut, uint32_t limit) {
+__device__ __forceinline__ void placeBlock(PlaceStage& s, const uint64_t (&key)[kPrefixItems], const uint32_t (&position)[kPrefixItems], uint32_t valid, uint32_t bins, int steps, uint32_t& cursor, PrefixRecord* __restrict__ out, uint32_t limit) {
     static_assert(kPrefixMaxBins == kPrefixThreads, "a bin per thread");
     const uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave;
     uint32_t place[kPrefixItems];  // bin, rank in the bin (below 4096)
@@ -506,8 +526,7 @@ __device__ __forceinline__ void placeBlock(PlaceStage& s, const uint64_t (&key)[
         if (x < total) {
             const uint32_t target = s.delta[s.bin[x]] + x;
             if (target < limit) {
-                keysOut[target] = s.key[x];
-                positionsOut[target] = s.position[x];
+                out[target] = packRecord(s.key[x], s.position[x]);
             }
         }
     }
@@ -517,7 +536,7 @@ __device__ __forceinline__ void placeBlock(PlaceStage& s, const uint64_t (&key)[
 // buckets), at (offsets[bucket * tiles + tile] - rowBase) onwards. The selected records of several
 // blocks collect in LDS until another block's might not fit, and are then placed together.
 template <class Texts>
-__global__ __launch_bounds__(kPrefixThreads, 4) void scatterBucketsKernel(PrefixText pt, Texts texts, CodeTable codes, const uint64_t* __restrict__ splitters, uint32_t allBuckets, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileBlocks, uint32_t tiles, const uint32_t* __restrict__ offsets, uint32_t rowBase, uint32_t limit, uint64_t* __restrict__ keysOut, uint32_t* __restrict__ positionsOut) {
+__global__ __launch_bounds__(kPrefixThreads, 4) void scatterBucketsKernel(PrefixText pt, Texts texts, CodeTable codes, const uint64_t* __restrict__ splitters, uint32_t allBuckets, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileBlocks, uint32_t tiles, const uint32_t* __restrict__ offsets, uint32_t rowBase, uint32_t limit, PrefixRecord* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char shared[];
     PlaceStage& stage = *reinterpret_cast<PlaceStage*>(shared);
     BlockCodes<Texts::kBatch>& s = *reinterpret_cast<BlockCodes<Texts::kBatch>*>(shared + (sizeof(PlaceStage) + 15) / 16 * 16);
@@ -545,7 +564,7 @@ __global__ __launch_bounds__(kPrefixThreads, 4) void scatterBucketsKernel(Prefix
             p[j] = stage.position[x];
             valid |= x < fill ? 1u << j : 0u;
         }
-        placeBlock(stage, k, p, valid, buckets, steps, cursor, keysOut, positionsOut, limit);
+        placeBlock(stage, k, p, valid, buckets, steps, cursor, out, limit);
         fill = 0;
         __syncthreads();
     };
@@ -655,7 +674,7 @@ __device__ __forceinline__ uint32_t bucketOfTile(const uint32_t* __restrict__ ti
 
 // Second level. A tile's counts lie at tilesBefore[bucket] * bins + bin * (tiles of the bucket) + (tile
 // in the bucket), so one exclusive sum gives every (bucket, bin, tile) its place in the round.
-__global__ __launch_bounds__(kPrefixThreads) void countBinsKernel(const uint64_t* __restrict__ keys, const uint64_t* __restrict__ splitters, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tilesBefore, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileRecords, uint32_t* __restrict__ counts) {
+__global__ __launch_bounds__(kPrefixThreads) void countBinsKernel(const PrefixRecord* __restrict__ records, const uint64_t* __restrict__ splitters, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tilesBefore, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileRecords, uint32_t* __restrict__ counts) {
     __shared__ uint64_t split[kPrefixMaxBins];
     __shared__ uint32_t histogram[kPrefixMaxBins];
     const uint32_t tile = xcdTile(blockIdx.x, gridDim.x);
@@ -675,7 +694,7 @@ __global__ __launch_bounds__(kPrefixThreads) void countBinsKernel(const uint64_t
         uint64_t key[kPrefixItems];
 #pragma unroll
         for (int j = 0; j < kPrefixItems; j++) {
-            key[j] = keys[min(x0 + j * kPrefixThreads, last - 1)];
+            key[j] = keyOf(records[min(x0 + j * kPrefixThreads, last - 1)]);
         }
 #pragma unroll
         for (int j = 0; j < kPrefixItems; j++) {
@@ -690,7 +709,7 @@ __global__ __launch_bounds__(kPrefixThreads) void countBinsKernel(const uint64_t
     }
 }
 
-__global__ __launch_bounds__(kPrefixThreads, 4) void scatterBinsKernel(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ positions, const uint64_t* __restrict__ splitters, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tilesBefore, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileRecords, const uint32_t* __restrict__ offsets, uint32_t limit, uint64_t* __restrict__ keysOut, uint32_t* __restrict__ positionsOut) {
+__global__ __launch_bounds__(kPrefixThreads, 4) void scatterBinsKernel(const PrefixRecord* __restrict__ records, const uint64_t* __restrict__ splitters, const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tilesBefore, uint32_t firstBucket, uint32_t buckets, uint32_t bins, int steps, uint32_t tileRecords, const uint32_t* __restrict__ offsets, uint32_t limit, PrefixRecord* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char shared[];
     PlaceStage& stage = *reinterpret_cast<PlaceStage*>(shared);
     const uint32_t tile = xcdTile(blockIdx.x, gridDim.x);
@@ -703,14 +722,11 @@ __global__ __launch_bounds__(kPrefixThreads, 4) void scatterBinsKernel(const uin
     const uint32_t last = min(starts[bucket + 1], first + tileRecords);
     const uint32_t t = threadIdx.x;
     // A block's records are loaded while the block before is placed.
-    uint64_t nextKey[kPrefixItems];
-    uint32_t nextPosition[kPrefixItems];
+    PrefixRecord next[kPrefixItems];
     auto load = [&](uint32_t block) {
 #pragma unroll
         for (int j = 0; j < kPrefixItems; j++) {
-            const uint32_t x = min(block + j * kPrefixThreads + t, last - 1);
-            nextKey[j] = keys[x];
-            nextPosition[j] = positions[x];
+            next[j] = records[min(block + j * kPrefixThreads + t, last - 1)];
         }
     };
     if (first < last) {
@@ -726,14 +742,14 @@ __global__ __launch_bounds__(kPrefixThreads, 4) void scatterBinsKernel(const uin
         uint32_t valid = 0;
 #pragma unroll
         for (int j = 0; j < kPrefixItems; j++) {
-            key[j] = nextKey[j];
-            position[j] = nextPosition[j];
+            key[j] = keyOf(next[j]);
+            position[j] = next[j].position;
             valid |= block + j * kPrefixThreads + t < last ? 1u << j : 0u;
         }
         if (block + kPrefixBlock < last) {
             load(block + kPrefixBlock);
         }
-        placeBlock(stage, key, position, valid, bins, steps, cursor, keysOut, positionsOut, limit);
+        placeBlock(stage, key, position, valid, bins, steps, cursor, out, limit);
     }
 }
 
@@ -770,8 +786,9 @@ struct RowOut {
 };
 
 // Row `row` (of all texts) holds `position`, whose record is `key`; tied: its key equals the row's
-// before, tiedNext: the row's after. The BWT bytes of tied rows are left to the tie kernels.
-__device__ __forceinline__ void emitRow(const RowOut& out, uint32_t row, uint64_t key, uint32_t position, bool tied, bool tiedNext) {
+// before. The BWT bytes of a group of tied rows wait in the group's places,
+// in the order of its positions (those of a text's suffix 0's own group: nowhere, they are read again).
+__device__ __forceinline__ void emitRow(const RowOut& out, uint32_t row, uint64_t key, uint32_t position, bool tied) {
     out.sa[row] = position;
     if (out.bwt) {
         const uint32_t segment = out.segmentBits ? static_cast<uint32_t>(key >> (64 - out.segmentBits)) : 0;
@@ -781,7 +798,7 @@ __device__ __forceinline__ void emitRow(const RowOut& out, uint32_t row, uint64_
             if (!tied) {
                 out.firstRows[segment] = row - out.segments[segment].rowBase;
             }
-        } else if (!tied && !tiedNext) {
+        } else {
             out.bwt[k < start ? row + 1 : row] = static_cast<uint8_t>(key);
         }
     }
@@ -822,10 +839,8 @@ constexpr int kLeafThreads = 256;
 constexpr int kLeafWaves = kLeafThreads / kWave;
 constexpr int kLeafLane = 8;                             // records a lane sorts in registers
 constexpr uint32_t kLeafChunk = kWave * kLeafLane;       // records a wave sorts in registers
-constexpr uint32_t kLeafChunks = kLeafCapacity / kLeafChunk;
 constexpr int kLeafIndexBits = 12;                       // of a record's index in its leaf
 constexpr uint32_t kLeafIndexMask = (1u << kLeafIndexBits) - 1;
-static_assert(kLeafCapacity == 1u << kLeafIndexBits && kLeafChunks == 2 * kLeafWaves, "two chunks a wave");
 
 // Lane l's value of lane l ^ kStride.
 template <int kStride>
@@ -935,15 +950,18 @@ __device__ __forceinline__ void mergeLeafRuns(uint64_t* values, uint32_t total, 
     __syncthreads();
 }
 
-// One workgroup per leaf of a round: keys[x] and out.sa[rowBase + x] for x in [leafStart[leaf],
-// leafStart[leaf + 1]), sorted by key in LDS and written to those rows. A leaf's keys share their
+// One workgroup per leaf of a group of buckets: records [leafStart[leaf], leafStart[leaf + 1]) sorted
+// by key in LDS and written to those rows past rowBase. A leaf's keys share their
 // upper bits, so the others and a record's index in the leaf fit one 64-bit value: a wave sorts 512
 // of them in registers (bitonic), and the sorted runs merge in LDS. Against LSD digit passes over
 // the records that is half the instructions, which is what bounds this kernel.
-__global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ leafStart, uint32_t rowBase, RowOut out, BigLeaves big) {
-    __shared__ uint64_t values[kLeafCapacity];
-    __shared__ uint32_t position[kLeafCapacity];
-    __shared__ uint8_t before[kLeafCapacity];
+template <uint32_t kCapacity>
+__global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRecord* __restrict__ records, const uint32_t* __restrict__ leafStart, uint32_t rowBase, RowOut out, BigLeaves big) {
+    static_assert(kCapacity <= 1u << kLeafIndexBits, "an index per record");
+    constexpr int kPasses = kCapacity / (kLeafChunk * kLeafWaves);  // chunks of a wave
+    __shared__ uint64_t values[kCapacity];
+    __shared__ uint32_t position[kCapacity];
+    __shared__ uint8_t before[kCapacity];
     __shared__ uint32_t differLow, differHigh;
 
     const uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave;
@@ -952,13 +970,17 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t*
     if (size == 0) {
         return;
     }
-    if (size > kLeafCapacity) {
+    if (size > kCapacity) {
         if (t == 0) {
             const uint32_t at = atomicAdd(&big.count[0], 1u);
             atomicAdd(&big.count[1], size);
             if (at < kBigLeavesMax) {
                 big.list[at] = uint2{rowBase + first, size};
             }
+        }
+        // Its positions wait in its rows, in any order.
+        for (uint32_t x = t; x < size; x += kLeafThreads) {
+            out.sa[rowBase + first + x] = records[first + x].position;
         }
         return;
     }
@@ -967,18 +989,20 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t*
         differHigh = 0;
     }
     const uint32_t chunks = (size + kLeafChunk - 1) / kLeafChunk;
-    const uint64_t reference = keys[first];
-    uint64_t key[2][kLeafLane];
+    records += first;
+    const uint64_t reference = keyOf(records[0]);
+    uint64_t key[kPasses][kLeafLane];
     uint64_t differ = 0;
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < kPasses; c++) {
         const uint32_t chunk = wave + c * kLeafWaves;
         if (chunk < chunks) {
 #pragma unroll
             for (int r = 0; r < kLeafLane; r++) {
                 const uint32_t x = min(chunk * kLeafChunk + r * kWave + lane, size - 1);
-                key[c][r] = keys[first + x];
-                position[x] = out.sa[rowBase + first + x];
+                const PrefixRecord record = records[x];
+                key[c][r] = keyOf(record);
+                position[x] = record.position;
             }
 #pragma unroll
             for (int r = 0; r < kLeafLane; r++) {
@@ -1005,7 +1029,7 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t*
     const bool truncated = shared < kLeafIndexBits - 8;
 
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
+    for (int c = 0; c < kPasses; c++) {
         const uint32_t chunk = wave + c * kLeafWaves;
         if (chunk < chunks) {
             uint64_t v[kLeafLane];
@@ -1031,36 +1055,36 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t*
     __syncthreads();
     if (differing) {
         for (uint32_t run = kLeafChunk; run < chunks * kLeafChunk; run *= 2) {
-            if (chunks <= kLeafWaves) {
-                mergeLeafRuns<kLeafCapacity / kLeafThreads / 2>(values, chunks * kLeafChunk, run);
+            if (kPasses == 1 || chunks <= kLeafWaves) {
+                mergeLeafRuns<kLeafLane>(values, chunks * kLeafChunk, run);
             } else {
-                mergeLeafRuns<kLeafCapacity / kLeafThreads>(values, chunks * kLeafChunk, run);
+                mergeLeafRuns<kLeafLane * kPasses>(values, chunks * kLeafChunk, run);
             }
         }
         if (truncated) {
             // Order each run of equal values by the four bits left out: a record's place is the number
             // of its run's records before it.
-            uint64_t moved[kLeafCapacity / kLeafThreads];
-            uint32_t target[kLeafCapacity / kLeafThreads];
+            uint64_t moved[kCapacity / kLeafThreads];
+            uint32_t target[kCapacity / kLeafThreads];
 #pragma unroll
-            for (uint32_t k = 0; k < kLeafCapacity / kLeafThreads; k++) {
+            for (uint32_t k = 0; k < kCapacity / kLeafThreads; k++) {
                 const uint32_t x = k * kLeafThreads + t;
                 target[k] = x;
                 if (x < size) {
                     const uint64_t v = values[leafSlot(x)];
                     moved[k] = v;
-                    const uint32_t own = static_cast<uint32_t>(keys[first + (v & kLeafIndexMask)]) & 0xF00u;
+                    const uint32_t own = records[v & kLeafIndexMask].low & 0xF00u;
                     for (uint32_t y = x; y-- > 0 && values[leafSlot(y)] >> kLeafIndexBits == v >> kLeafIndexBits;) {
-                        target[k] -= (static_cast<uint32_t>(keys[first + (values[leafSlot(y)] & kLeafIndexMask)]) & 0xF00u) > own ? 1 : 0;
+                        target[k] -= (records[values[leafSlot(y)] & kLeafIndexMask].low & 0xF00u) > own ? 1 : 0;
                     }
                     for (uint32_t y = x + 1; y < size && values[leafSlot(y)] >> kLeafIndexBits == v >> kLeafIndexBits; y++) {
-                        target[k] += (static_cast<uint32_t>(keys[first + (values[leafSlot(y)] & kLeafIndexMask)]) & 0xF00u) < own ? 1 : 0;
+                        target[k] += (records[values[leafSlot(y)] & kLeafIndexMask].low & 0xF00u) < own ? 1 : 0;
                     }
                 }
             }
             __syncthreads();
 #pragma unroll
-            for (uint32_t k = 0; k < kLeafCapacity / kLeafThreads; k++) {
+            for (uint32_t k = 0; k < kCapacity / kLeafThreads; k++) {
                 if (k * kLeafThreads + t < size) {
                     values[leafSlot(target[k])] = moved[k];
                 }
@@ -1074,18 +1098,16 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const uint64_t*
         const bool valid = x < size;
         const uint64_t v = values[leafSlot(min(x, size - 1))];
         const uint32_t index = static_cast<uint32_t>(v) & kLeafIndexMask;
-        const uint64_t previous = values[leafSlot(x > 0 && valid ? x - 1 : 0)], next = values[leafSlot(min(x + 1, size - 1))];
+        const uint64_t previous = values[leafSlot(x > 0 && valid ? x - 1 : 0)];
         bool tied = valid && x > 0 && previous >> kLeafIndexBits == v >> kLeafIndexBits;
-        bool tiedNext = x + 1 < size && next >> kLeafIndexBits == v >> kLeafIndexBits;
         uint64_t key = differing ? top | (v & ~static_cast<uint64_t>(kLeafIndexMask)) >> shared : top;
         if (truncated) {
-            const uint32_t own = static_cast<uint32_t>(keys[first + index]) & 0xF00u;
+            const uint32_t own = records[index].low & 0xF00u;
             key |= own;
-            tied = tied && (static_cast<uint32_t>(keys[first + (previous & kLeafIndexMask)]) & 0xF00u) == own;
-            tiedNext = tiedNext && (static_cast<uint32_t>(keys[first + (next & kLeafIndexMask)]) & 0xF00u) == own;
+            tied = tied && (records[previous & kLeafIndexMask].low & 0xF00u) == own;
         }
         if (valid) {
-            emitRow(out, rowBase + first + x, key | before[index], position[index], tied, tiedNext);
+            emitRow(out, rowBase + first + x, key | before[index], position[index], tied);
         }
         emitTies(out.ties, rowBase + first + x - lane, ballot(tied));
     }
@@ -1124,8 +1146,7 @@ __global__ __launch_bounds__(256) void bigLeafRowsKernel(const uint64_t* __restr
     const uint32_t row = list[leaf].x + (k - before[leaf]);
     const uint64_t key = keys[k];
     const bool tied = k > 0 && keyPart(keys[k - 1]) == keyPart(key);
-    const bool tiedNext = k + 1 < total && keyPart(keys[k + 1]) == keyPart(key);
-    emitRow(out, row, key, positions[k], tied, tiedNext);
+    emitRow(out, row, key, positions[k], tied);
     if (tied) {
         atomicOr(&out.ties[row >> 5], 1u << (row & 31));
     }
@@ -1287,81 +1308,166 @@ struct TieConsumer {
     }
 };
 
-// A tied row's final place: the position at `row` of the suffix array and the character before it.
-template <class Texts>
-__device__ __forceinline__ void placeTied(const MergeCtx& c, const Texts& texts, const RowOut& out, uint32_t row, uint32_t position, uint32_t before, uint32_t startLocal) {
-    out.sa[row] = position;
-    if (out.bwt) {
-        const uint32_t segment = texts.segmentOf(position);
-        const uint32_t start = texts.startOf(position);
-        const uint32_t local = row - out.segments[segment].rowBase;
-        if (position == start) {
-            out.firstRows[segment] = local;
-        } else {
-            out.bwt[local < startLocal ? row + 1 : row] = static_cast<uint8_t>(before);
-        }
-    }
-}
-
 constexpr uint32_t kTieTile = 256;
 constexpr uint32_t kTieRecords = kTieTile + kTieGroupMax;
 
+constexpr int kTieRounds = (kTieRecords + kTieTile - 1) / kTieTile;  // list entries of a thread
+using RankQuad = uint32_t __attribute__((ext_vector_type(4), aligned(4)));
+
 // Groups of up to kTieGroupMax rows whose first row is in the workgroup's part of the list: every
 // member's place is the number of members smaller than it. Members of larger groups are flagged.
+//
+// Two suffixes i and j compare at the smallest offset k with i + k and j + k both sampled: the
+// characters before it, then the ranks there. Bound by the random lines this reads, so a member reads
+// the one rank of a pair (the window of seven in a larger group), and its text only if some k of its
+// group lies past the `shared` characters of the group's key; the comparisons are between copies in LDS.
 template <class Texts>
-__global__ __launch_bounds__(kTieTile) void tieGroupsKernel(MergeCtx c, Texts texts, const uint32_t* __restrict__ rows, uint32_t count, RowOut out, uint8_t* __restrict__ large, uint32_t* __restrict__ largeCount) {
-    extern __shared__ __align__(16) unsigned char shared[];
-    LdsRecords<32, Texts::kBatch> recs;
-    recs.carve(shared, kTieRecords);
+__global__ __launch_bounds__(kTieTile) void tieGroupsKernel(MergeCtx c, Texts texts, uint32_t shared, const uint32_t* __restrict__ rows, uint32_t count, RowOut out, uint8_t* __restrict__ large, uint32_t* __restrict__ largeCount) {
+    constexpr int kRanks = CoverSet<32>::kSize;
     __shared__ uint32_t listed[kTieGroupMax + kTieRecords + 1];  // rows from kTieGroupMax before the tile
-    __shared__ uint8_t before[kTieRecords];
-    __shared__ uint8_t headOf[kTieRecords], sizeOf[kTieRecords];  // distance back to the head; group size, 0 if not handled here
+    __shared__ uint32_t position[kTieRecords];
+    __shared__ uint32_t ranks[kRanks][kTieRecords];  // the window's, or the pair's in ranks[0]
+    __shared__ uint64_t words[4][kTieRecords];       // characters from shared & ~7 on
     const uint32_t tile0 = blockIdx.x * kTieTile;
     for (uint32_t x = threadIdx.x; x < kTieGroupMax + kTieRecords + 1; x += kTieTile) {
         const int64_t j = static_cast<int64_t>(tile0) + x - kTieGroupMax;
-        listed[x] = j >= 0 && j < count ? rows[j] : kTieHead;
+        const uint32_t row = j >= 0 && j < count ? rows[j] : kTieHead;
+        listed[x] = row;
+        if (x >= kTieGroupMax && x < kTieGroupMax + kTieRecords && j < count) {
+            const uint32_t p = out.sa[row & ~kTieHead];
+            position[x - kTieGroupMax] = p < c.n ? p : 0;
+        }
     }
     __syncthreads();
     const uint32_t inList = min(kTieRecords, count - tile0);  // entries of the tile and after it
+    const uint32_t firstChar = shared & ~7u;
+    auto offsetOf = [](uint32_t i, uint32_t j) -> uint32_t {
+        return __builtin_ctz(windowOf32(coverMask<32>(), i) & windowOf32(coverMask<32>(), j));
+    };
+    uint32_t head[kTieRounds], size[kTieRounds];  // of the entry's group, size 0 if it is not handled here
     uint32_t flagged = 0;
-    for (uint32_t x = threadIdx.x; x < kTieRecords; x += kTieTile) {
-        uint32_t size = 0, back = 0;
-        if (x < inList) {
-            while (back <= kTieGroupMax && x + kTieGroupMax >= back && !(listed[x + kTieGroupMax - back] & kTieHead)) {
-                back++;
-            }
-            // back <= kTieGroupMax: the head is listed[x + kTieGroupMax - back]. Past the list's ends
-            // every entry is a head.
-            if (back < kTieGroupMax) {
-                const uint32_t head = x + kTieGroupMax - back;
-                size = back + 1;
-                while (size <= kTieGroupMax && head + size < kTieGroupMax + kTieRecords + 1 && !(listed[head + size] & kTieHead)) {
-                    size++;
-                }
-            } else {
-                size = kTieGroupMax + 1;
-            }
-            if (x < kTieTile) {
-                const bool isLarge = size > kTieGroupMax;
-                large[tile0 + x] = isLarge ? 1 : 0;
-                flagged += isLarge ? 1 : 0;
-            }
-            // Handled here: small, the head in the tile.
-            if (size > kTieGroupMax || back > x || x - back >= kTieTile) {
-                size = 0;
+#pragma unroll
+    for (int round = 0; round < kTieRounds; round++) {
+        const uint32_t x = threadIdx.x + round * kTieTile;
+        head[round] = 0;
+        size[round] = 0;
+        if (x >= inList) {
+            continue;
+        }
+        uint32_t back = 0;
+        while (back <= kTieGroupMax && !(listed[x + kTieGroupMax - back] & kTieHead)) {
+            back++;
+        }
+        // back < kTieGroupMax: the head is listed[x + kTieGroupMax - back]. Past the list's ends every
+        // entry is a head.
+        uint32_t length = kTieGroupMax + 1;
+        if (back < kTieGroupMax) {
+            const uint32_t first = x + kTieGroupMax - back;
+            length = back + 1;
+            while (length <= kTieGroupMax && first + length < kTieGroupMax + kTieRecords + 1 && !(listed[first + length] & kTieHead)) {
+                length++;
             }
         }
-        headOf[x] = static_cast<uint8_t>(back);
-        sizeOf[x] = static_cast<uint8_t>(size);
-        if (size) {
-            const uint32_t row = listed[x + kTieGroupMax] & ~kTieHead;
-            uint32_t p = out.sa[row];
-            p = p < c.n ? p : 0;
-            MergeRecord<32, Texts::kBatch> record;
-            uint8_t characterBefore;
-            loadRecord<32, Texts>(c, texts, p, record, &characterBefore);
-            recs.store(x, record);
-            before[x] = characterBefore;
+        if (x < kTieTile) {
+            const bool isLarge = length > kTieGroupMax;
+            large[tile0 + x] = isLarge ? 1 : 0;
+            flagged += isLarge ? 1 : 0;
+        }
+        // Handled here: small, the head in the tile.
+        if (length > kTieGroupMax || back > x || x - back >= kTieTile) {
+            continue;
+        }
+        head[round] = x - back;
+        size[round] = length;
+        const uint32_t p = position[x];
+        uint32_t furthest = 0;
+        for (uint32_t y = x - back; y < x - back + length; y++) {
+            furthest = y != x ? max(furthest, offsetOf(p, position[y])) : furthest;
+        }
+        if (length == 2) {
+            ranks[0][x] = p + furthest < texts.endOf(p) ? c.ranks[packPosition<32>(p + furthest)] : 0;
+        } else {
+            const uint32_t* window = c.ranks + (p / 32) * kRanks + coverBelow<32>(p & 31);
+            const RankQuad a = *reinterpret_cast<const RankQuad*>(window), b = *reinterpret_cast<const RankQuad*>(window + 3);
+            ranks[0][x] = a.x;
+            ranks[1][x] = a.y;
+            ranks[2][x] = a.z;
+            ranks[3][x] = a.w;
+            ranks[4][x] = b.y;
+            ranks[5][x] = b.z;
+            ranks[6][x] = b.w;
+        }
+        if (furthest > shared) {
+            const uint32_t at = p + firstChar, shift = (at & 7) * 8;
+            uint64_t low = c.text[at >> 3];
+#pragma unroll
+            for (uint32_t w = 0; w < 4; w++) {
+                if (firstChar + 8 * w < 32) {
+                    const uint64_t high = c.text[(at >> 3) + w + 1];
+                    words[w][x] = __builtin_bswap64(shift ? (low >> shift) | (high << (64 - shift)) : low);
+                    low = high;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t target[kTieRounds], byteAt[kTieRounds];
+    uint8_t byte[kTieRounds];
+#pragma unroll
+    for (int round = 0; round < kTieRounds; round++) {
+        const uint32_t x = threadIdx.x + round * kTieTile;
+        if (size[round] == 0) {
+            continue;
+        }
+        const uint32_t p = position[x], end = texts.endOf(p), start = texts.startOf(p);
+        const uint32_t headRow = listed[head[round] + kTieGroupMax] & ~kTieHead;
+        uint32_t smaller = 0;
+        bool startHere = p == start, afterStart = false;
+        for (uint32_t y = head[round]; y < head[round] + size[round]; y++) {
+            if (y == x) {
+                continue;
+            }
+            const uint32_t q = position[y];
+            const uint32_t k = offsetOf(p, q);
+            const uint32_t last = max(p, q);
+            const uint32_t common = min(k, end - last);
+            bool less = q > p, decided = false;  // one a prefix of the other: the shorter is smaller
+            if (common > shared) {
+#pragma unroll
+                for (uint32_t w = 0; w < 4; w++) {
+                    const uint32_t from = firstChar + 8 * w;
+                    if (from < common && !decided) {
+                        const uint64_t mask = prefixMask(common - from);
+                        const uint64_t own = words[w][x] & mask, other = words[w][y] & mask;
+                        decided = own != other;
+                        less = decided ? other < own : less;
+                    }
+                }
+            }
+            if (!decided && last + k < end) {
+                const uint32_t before = (1u << k) - 1;
+                const uint32_t ownSlot = size[round] == 2 ? 0 : __builtin_popcount(windowOf32(coverMask<32>(), p) & before);
+                const uint32_t otherSlot = size[round] == 2 ? 0 : __builtin_popcount(windowOf32(coverMask<32>(), q) & before);
+                less = ranks[otherSlot][y] < ranks[ownSlot][x];
+            }
+            smaller += less ? 1 : 0;
+            if (q == start) {
+                startHere = true;
+                afterStart = less;
+            }
+        }
+        target[round] = headRow + smaller;
+        if (out.bwt) {
+            const uint32_t segment = texts.segmentOf(p);
+            if (!startHere) {
+                // The group's bytes are in its own places, one further on before the text's first row.
+                const uint32_t shift = headRow - out.segments[segment].rowBase < out.firstRows[segment] ? 1 : 0;
+                byte[round] = out.bwt[headRow + (x - head[round]) + shift];
+                byteAt[round] = headRow + smaller + shift;
+            } else {
+                byte[round] = p != start ? reinterpret_cast<const uint8_t*>(c.text)[p - 1] : 0;
+                byteAt[round] = headRow + smaller + (afterStart ? 0 : 1);
+            }
         }
     }
     const uint64_t any = ballot(flagged != 0);
@@ -1373,32 +1479,21 @@ __global__ __launch_bounds__(kTieTile) void tieGroupsKernel(MergeCtx c, Texts te
             atomicAdd(largeCount, flagged);
         }
     }
+    // Every byte of the tile's groups is read before any is written.
     __syncthreads();
-    const TieTables tables{nullptr, nullptr};
-    for (uint32_t x = threadIdx.x; x < kTieRecords; x += kTieTile) {
-        const uint32_t size = sizeOf[x];
-        if (size) {
-            const uint32_t head = x - headOf[x];
-            const uint32_t headRow = listed[head + kTieGroupMax] & ~kTieHead;
-            const uint32_t p = recs.positionOf(x);
-            uint32_t smaller = 0, startLocal = 0;
-            const uint32_t segment = texts.segmentOf(p), start = texts.startOf(p);
-            bool startHere = false;
-            uint32_t startEntry = 0;
-            for (uint32_t y = head; y < head + size; y++) {
-                smaller += y != x && lessLds<32, Texts>(c, tables, recs, y, x) ? 1 : 0;
-                if (recs.positionOf(y) == start) {
-                    startHere = true;
-                    startEntry = y;
+#pragma unroll
+    for (int round = 0; round < kTieRounds; round++) {
+        if (size[round]) {
+            const uint32_t p = position[threadIdx.x + round * kTieTile];
+            out.sa[target[round]] = p;
+            if (out.bwt) {
+                if (p == texts.startOf(p)) {
+                    const uint32_t segment = texts.segmentOf(p);
+                    out.firstRows[segment] = target[round] - out.segments[segment].rowBase;
+                } else {
+                    out.bwt[byteAt[round]] = byte[round];
                 }
             }
-            if (out.bwt) {
-                // In the group of suffix 0 itself, the rows before it are those of smaller members.
-                const uint32_t local = headRow + smaller - out.segments[segment].rowBase;
-                startLocal = !startHere ? out.firstRows[segment]
-                           : startEntry != x && lessLds<32, Texts>(c, tables, recs, x, startEntry) ? local + 1 : local;
-            }
-            placeTied(c, texts, out, headRow + smaller, p, before[x], startLocal);
         }
     }
 }
@@ -1502,12 +1597,33 @@ __global__ __launch_bounds__(256) void largeBytesKernel(MergeCtx c, Texts texts,
     }
 }
 
-// A batch's rows hold positions of all texts; the outputs are positions in each text.
-template <class Texts>
-__global__ __launch_bounds__(256) void localRowsKernel(Texts texts, uint32_t* __restrict__ sa, uint32_t count) {
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < count; r += gridDim.x * blockDim.x) {
-        const uint32_t p = sa[r];
-        sa[r] = p - texts.startOf(p);
+// A batch's rows hold positions of all texts; the outputs are positions in each text. A workgroup's
+// rows are consecutive, mostly of one text: it searches the row's text once and steps from there (a
+// lookup by position reads two tables at random for every row: 2.9 against 1.1 ms for 515M rows).
+constexpr int kLocalItems = 16;
+
+__global__ __launch_bounds__(256) void localRowsKernel(const Segment* __restrict__ segments, uint32_t texts, uint32_t* __restrict__ sa, uint32_t count) {
+    const uint64_t first = static_cast<uint64_t>(blockIdx.x) * 256 * kLocalItems;
+    uint32_t lo = 0, hi = texts;  // the last text with rowBase <= first
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (segments[mid].rowBase <= first) {
+            lo = mid;
+        } else {
+            hi = mid;
+        }
+    }
+    uint32_t text = lo;
+    Segment segment = segments[text];
+#pragma unroll
+    for (int j = 0; j < kLocalItems; j++) {
+        const uint64_t row = first + j * 256 + threadIdx.x;
+        if (row < count) {
+            while (row >= segment.rowBase + static_cast<uint64_t>(segment.end - segment.start)) {
+                segment = segments[++text];
+            }
+            sa[row] -= segment.start;
+        }
     }
 }
 
