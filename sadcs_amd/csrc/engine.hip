@@ -1170,7 +1170,7 @@ class Pipeline {
         // Buckets and leaves.
         // Few leaves: larger ones from a smaller sample, which sorts by counting.
         const bool coarse = N <= static_cast<uint64_t>(kSampleCountMax) * kCoarseLeaf / kCoarseOversample;
-        const uint32_t leafTarget = coarse ? kCoarseLeaf : kLeafTarget;
+        const uint32_t leafTarget = coarse ? std::clamp<uint32_t>(static_cast<uint32_t>(N / kPrefixMaxRoundBuckets), kSmallLeaf, kCoarseLeaf) : kLeafTarget;
         const uint64_t leavesWanted = std::min<uint64_t>((N + leafTarget - 1) / leafTarget, static_cast<uint64_t>(kPrefixMaxBuckets) * kPrefixMaxBins);
         uint32_t buckets = 1, bins = 1;
         if (N > kLeafCapacity) {
@@ -1365,11 +1365,8 @@ class Pipeline {
             return SADCS_OK;
         }
 
-        fillWords(out.ties, tieWords + 4, 0);
-        if (out.bwt) {
-            startKeysKernel<Texts><<<blocksFor(m_segments), 256, 0, m_stream>>>(pt, m_texts, codes, m_job.deviceSegments, m_segments, startKeys);
-            firstBwtBytesKernel<<<blocksFor(m_segments), 256, 0, m_stream>>>(m_job.text, m_job.deviceSegments, m_segments, out.bwt);
-        }
+        initRowsKernel<Texts><<<std::min<unsigned>(blocksFor(std::max<uint64_t>(m_segments, tieWords + 4)), 4096), 256, 0, m_stream>>>(
+            pt, m_texts, codes, m_job.deviceSegments, m_segments, startKeys, out.ties, tieWords + 4, out.bwt);
 
         // The records a round holds and, two levels, a group of its buckets' records again and counts.
         const uint32_t maxRoundBuckets = std::min(buckets, kPrefixMaxRoundBuckets);
@@ -1447,18 +1444,21 @@ class Pipeline {
                     continue;
                 }
                 const uint32_t groupBase = rows[g.first];
-                bucketTilesKernel<<<1, kPrefixMaxRoundBuckets, 0, m_stream>>>(offsets, tiles, buckets, g.first, g.count, rowBase, static_cast<uint32_t>(N), tileRecords, starts, tilesBefore);
                 if (bins > 1) {
                     const uint32_t groupTiles = g.rows / tileRecords + g.count + 1;
                     const int binSteps = log2Ceil(bins);
+                    bucketTilesKernel<<<1, kPrefixMaxRoundBuckets, 0, m_stream>>>(offsets, tiles, buckets, g.first, g.count, rowBase, static_cast<uint32_t>(N), tileRecords, starts, tilesBefore);
                     countBinsKernel<<<groupTiles, kPrefixThreads, 0, m_stream>>>(recordsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords, binOffsets);
                     exclusiveSum(m_stream, binOffsets, binOffsets, groupTiles * bins, binAggregates);
                     scatterBinsKernel<<<groupTiles, kPrefixThreads, binShared, m_stream>>>(recordsA, splitters, starts, tilesBefore, g.first, g.count, bins, binSteps, tileRecords,
                                                                                           binOffsets, g.rows, recordsB);
+                    leafStartsKernel<<<blocksFor(static_cast<uint64_t>(g.count) * bins + 1), 256, 0, m_stream>>>(starts, tilesBefore, binOffsets, g.count, bins, leafStart);
                 }
-                leafStartsKernel<<<blocksFor(static_cast<uint64_t>(g.count) * bins + 1), 256, 0, m_stream>>>(starts, tilesBefore, binOffsets, g.count, bins, leafStart);
+                // One level: the buckets are the leaves, and tableRows their first rows.
+                const uint32_t* leafRows = bins > 1 ? leafStart : tableRows + g.first;
+                const uint32_t leafBase = bins > 1 ? 0 : groupBase;
                 const auto sortLeaves = N > static_cast<uint64_t>(leaves) * kLeafTarget ? sortLeavesKernel<2 * kLeafCapacity> : sortLeavesKernel<kLeafCapacity>;
-                sortLeaves<<<g.count * bins, kLeafThreads, 0, m_stream>>>(bins > 1 ? recordsB : recordsA, leafStart, groupBase, out, big);
+                sortLeaves<<<g.count * bins, kLeafThreads, 0, m_stream>>>(bins > 1 ? recordsB : recordsA, leafRows, leafBase, groupBase, out, big);
                 SADCS_HIP(hipGetLastError());
             }
         }
@@ -1562,20 +1562,30 @@ class Pipeline {
             releaseTaken();
             return SADCS_OK;
         }
-        fillWords(m_ranks, rankWords, 0);
+        // Every sample position gets its rank below; what lies between a batch's texts and past the last
+        // is read beside ranks but not used.
         scanPipeline<SampleVec, kSampleItems>(m_stream, N, SampleProducer<V>{out.sa, out.ties}, SampleConsumer<V>{out.sa, index, group, M}, sampleAggregates);
         const GroupProducer groups{group, M};
-        const uint32_t groupTiles = std::max<uint32_t>(1, ceilDiv(M, uint64_t(kScanThreads) * kMarkItems));
-        scanReduceKernel<GroupVec, kMarkItems><<<groupTiles, kScanThreads, 0, m_stream>>>(groups, M, groupAggregates);
-        scanAggregatesKernel<GroupVec><<<1, kScanThreads, 0, m_stream>>>(groupAggregates, groupTiles);
-        const uint32_t tieTiles = std::max<uint32_t>(1, ceilDiv(tieWords, uint64_t(kScanThreads) * kSumItems));
-        scanReduceKernel<Sum1, kSumItems><<<tieTiles, kScanThreads, 0, m_stream>>>(TieProducer{out.ties}, tieWords, tieAggregates);
-        scanAggregatesKernel<Sum1><<<1, kScanThreads, 0, m_stream>>>(tieAggregates, tieTiles);
-        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, groupAggregates + groupTiles, sizeof(GroupVec), hipMemcpyDeviceToHost, m_stream));
-        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords + 4, tieAggregates + tieTiles, sizeof(Sum1), hipMemcpyDeviceToHost, m_stream));
+        scanReduce<GroupVec, kMarkItems>(m_stream, M, groups, groupAggregates);
+        scanReduce<Sum1, kSumItems>(m_stream, tieWords, TieProducer{out.ties}, tieAggregates);
+        SADCS_HIP(hipGetLastError());
+        // The totals: past the scanned aggregates, or the sums of a few tiles' own.
+        GroupVec* groupHost = reinterpret_cast<GroupVec*>(m_ctx.hostWords);
+        Sum1* tieHost = reinterpret_cast<Sum1*>(m_ctx.hostWords + 1024);
+        const uint32_t groupTiles = scanTiles<kMarkItems>(M), tieTiles = scanTiles<kSumItems>(tieWords);
+        const bool groupFew = groupTiles <= kScanThreads, tieFew = tieTiles <= kScanThreads;
+        SADCS_HIP(hipMemcpyAsync(groupHost, groupAggregates + (groupFew ? 0 : groupTiles), (groupFew ? groupTiles : 1) * sizeof(GroupVec), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipMemcpyAsync(tieHost, tieAggregates + (tieFew ? 0 : tieTiles), (tieFew ? tieTiles : 1) * sizeof(Sum1), hipMemcpyDeviceToHost, m_stream));
         SADCS_HIP(hipStreamSynchronize(m_stream));
-        const uint32_t unresolved = m_ctx.hostWords[1], unresolvedGroups = m_ctx.hostWords[2];
-        tied = m_ctx.hostWords[4];
+        uint32_t unresolved = 0, unresolvedGroups = 0;
+        for (uint32_t x = 0; x < (groupFew ? groupTiles : 1); x++) {
+            unresolved += groupHost[x].v[1];
+            unresolvedGroups += groupHost[x].v[2];
+        }
+        tied = 0;
+        for (uint32_t x = 0; x < (tieFew ? tieTiles : 1); x++) {
+            tied += tieHost[x].v[0];
+        }
 
         RankPassState state;
         if (unresolved > 0) {
@@ -1584,8 +1594,8 @@ class Pipeline {
                 releaseTaken();
                 return SADCS_OK;
             }
-            scanDownsweepKernel<GroupVec, kMarkItems><<<groupTiles, kScanThreads, 0, m_stream>>>(
-                groups, GroupConsumer{index, m_ranks, state.values[1], reinterpret_cast<uint32_t*>(state.keys[1]), state.groupIds[0]}, M, groupAggregates);
+            scanDownsweep<GroupVec, kMarkItems>(
+                m_stream, M, groups, GroupConsumer{index, m_ranks, state.values[1], reinterpret_cast<uint32_t*>(state.keys[1]), state.groupIds[0]}, groupAggregates);
         }
         const uint32_t rankCount = static_cast<uint32_t>(DifferenceCover<V>::pack(m_job.span));
         const uint64_t windows = std::max<uint64_t>(1, (uint64_t(rankCount) * sizeof(uint32_t) + kDeferredRankWindow - 1) / kDeferredRankWindow);
@@ -2369,7 +2379,12 @@ size_t planBytes(const sadcs_ctx& base, const Layout& layout, Mode mode, bool ow
         std::unique_ptr<Pipeline<V, SingleText>> keep;
         status = runPipeline<V, SingleText>(ctx, job, SingleText{layout.span}, times, nullptr, nullptr, keep);
     }
-    return status == SADCS_OK ? ctx.arena.highWater() : SIZE_MAX;
+    if (status != SADCS_OK) {
+        return SIZE_MAX;
+    }
+    // A text below 1 MiB is bound by launches, not by memory: room for the prefix sort in one round.
+    const size_t roomy = mode != Mode::RankOnly && layout.span < (uint32_t(1) << 20) ? size_t(1) << 19 : 0;
+    return std::max(ctx.arena.highWater(), roomy ? roomy + (ownOutputs ? 32 : 26) * static_cast<size_t>(layout.span) : 0);
 }
 
 size_t planFor(const sadcs_ctx& base, const Layout& layout, Mode mode, bool ownText, bool ownOutputs) {

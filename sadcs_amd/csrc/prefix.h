@@ -51,7 +51,9 @@ constexpr uint32_t kPrefixMaxBins = 512;           // leaves of a bucket
 constexpr uint32_t kLeafTarget = 1024;
 constexpr uint32_t kLeafCapacity = 2048;
 constexpr uint32_t kOversample = 32;
-// Up to about 2.3 million rows: leaves of 1536 on average, of up to 4096, from 16 keys a leaf.
+// Up to about 2.3 million rows: leaves of 512 to 1536 on average (about 512 of them while that
+// holds: every CU has leaves to sort, and a small one sorts sooner), of up to 4096, 16 keys a leaf.
+constexpr uint32_t kSmallLeaf = 512;
 constexpr uint32_t kCoarseLeaf = 1536;
 constexpr uint32_t kCoarseOversample = 16;
 constexpr uint32_t kTieGroupMax = 24;              // rows of a group compared in LDS
@@ -753,8 +755,7 @@ __global__ __launch_bounds__(kPrefixThreads, 4) void scatterBinsKernel(const Pre
     }
 }
 
-// leafStart[x] of a group of buckets: the first record of leaf x in it (x = leaves: the total). One
-// level (bins = 1): from the buckets' starts; two: from the bins' offsets.
+// leafStart[x] of a group of buckets: the first record of leaf x in it (x = leaves: the total).
 __global__ __launch_bounds__(256) void leafStartsKernel(const uint32_t* __restrict__ starts, const uint32_t* __restrict__ tilesBefore, const uint32_t* __restrict__ offsets, uint32_t buckets, uint32_t bins, uint32_t* __restrict__ leafStart) {
     const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
     if (x > buckets * bins) {
@@ -762,8 +763,6 @@ __global__ __launch_bounds__(256) void leafStartsKernel(const uint32_t* __restri
     }
     if (x == buckets * bins) {
         leafStart[x] = starts[buckets] - starts[0];
-    } else if (bins == 1) {
-        leafStart[x] = starts[x] - starts[0];
     } else {
         const uint32_t b = x / bins, before = tilesBefore[b], tilesHere = tilesBefore[b + 1] - before;
         leafStart[x] = offsets[static_cast<uint64_t>(before) * bins + static_cast<uint64_t>(x % bins) * tilesHere];
@@ -818,13 +817,21 @@ __device__ __forceinline__ void emitTies(uint32_t* __restrict__ ties, uint32_t r
     }
 }
 
+// Before the rows are written: no ties, the texts' start keys, and with a BWT byte 0 of every text,
+// T[end - 1].
 template <class Texts>
-__global__ void startKeysKernel(PrefixText pt, Texts texts, CodeTable codes, const Segment* __restrict__ segments, uint32_t count, uint64_t* __restrict__ startKeys) {
+__global__ __launch_bounds__(256) void initRowsKernel(PrefixText pt, Texts texts, CodeTable codes, const Segment* __restrict__ segments, uint32_t count, uint64_t* __restrict__ startKeys, uint32_t* __restrict__ ties, uint32_t tieWords, uint8_t* __restrict__ bwt) {
     __shared__ uint8_t code[256];
     loadCodes(codes, code);
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < count) {
+    const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (uint32_t w = first; w < tieWords; w += stride) {
+        ties[w] = 0;
+    }
+    for (uint32_t s = first; s < count; s += stride) {
         startKeys[s] = prefixKey(pt, texts, code, segments[s].start);
+        if (bwt) {
+            bwt[segments[s].rowBase] = reinterpret_cast<const uint8_t*>(pt.words)[segments[s].end - 1];
+        }
     }
 }
 
@@ -950,13 +957,13 @@ __device__ __forceinline__ void mergeLeafRuns(uint64_t* values, uint32_t total, 
     __syncthreads();
 }
 
-// One workgroup per leaf of a group of buckets: records [leafStart[leaf], leafStart[leaf + 1]) sorted
-// by key in LDS and written to those rows past rowBase. A leaf's keys share their
+// One workgroup per leaf of a group of buckets: records [leafStart[leaf], leafStart[leaf + 1]) less
+// leafBase, sorted by key in LDS and written to those rows past rowBase. A leaf's keys share their
 // upper bits, so the others and a record's index in the leaf fit one 64-bit value: a wave sorts 512
 // of them in registers (bitonic), and the sorted runs merge in LDS. Against LSD digit passes over
 // the records that is half the instructions, which is what bounds this kernel.
 template <uint32_t kCapacity>
-__global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRecord* __restrict__ records, const uint32_t* __restrict__ leafStart, uint32_t rowBase, RowOut out, BigLeaves big) {
+__global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRecord* __restrict__ records, const uint32_t* __restrict__ leafStart, uint32_t leafBase, uint32_t rowBase, RowOut out, BigLeaves big) {
     static_assert(kCapacity <= 1u << kLeafIndexBits, "an index per record");
     constexpr int kPasses = kCapacity / (kLeafChunk * kLeafWaves);  // chunks of a wave
     __shared__ uint64_t values[kCapacity];
@@ -965,8 +972,8 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
     __shared__ uint32_t differLow, differHigh;
 
     const uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave;
-    const uint32_t first = leafStart[blockIdx.x];
-    const uint32_t size = leafStart[blockIdx.x + 1] - first;
+    const uint32_t first = leafStart[blockIdx.x] - leafBase;
+    const uint32_t size = leafStart[blockIdx.x + 1] - leafBase - first;
     if (size == 0) {
         return;
     }

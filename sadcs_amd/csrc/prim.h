@@ -146,9 +146,12 @@ __global__ __launch_bounds__(kScanThreads) void scanAggregatesKernel(VecT* __res
     }
 }
 
-template <class VecT, int ITEMS, class Producer, class Consumer>
-__global__ __launch_bounds__(kScanThreads) void scanDownsweepKernel(Producer produce, Consumer consume, uint32_t count, const VecT* __restrict__ aggregates) {
+// kRaw: the aggregates are the tiles' own, at most kScanThreads of them; every workgroup combines those
+// before it (a launch less than scanning them first), and the last one leaves the total past them.
+template <class VecT, int ITEMS, bool kRaw, class Producer, class Consumer>
+__global__ __launch_bounds__(kScanThreads) void scanDownsweepKernel(Producer produce, Consumer consume, uint32_t count, VecT* __restrict__ aggregates) {
     __shared__ VecT waveTotals[kScanWaves];
+    __shared__ VecT before[kScanWaves];
     const uint32_t wave = threadIdx.x / kWave;
     const uint32_t lane = threadIdx.x % kWave;
     const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScanThreads * ITEMS + wave * ITEMS * kWave + lane;
@@ -175,9 +178,30 @@ __global__ __launch_bounds__(kScanThreads) void scanDownsweepKernel(Producer pro
     if (lane == 0) {
         waveTotals[wave] = carry;
     }
+    if constexpr (kRaw) {
+        VecT own = threadIdx.x < blockIdx.x ? aggregates[threadIdx.x] : VecT::zero();
+        own = VecT::lane(VecT::waveInclusive(own), kWave - 1);
+        if (lane == 0) {
+            before[wave] = own;
+        }
+    }
     __syncthreads();
 
-    VecT prefix = aggregates[blockIdx.x];
+    VecT prefix = VecT::zero();
+    if constexpr (kRaw) {
+        for (int w = 0; w < kScanWaves; w++) {
+            prefix = VecT::combine(prefix, before[w]);
+        }
+        if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) {
+            VecT total = prefix;
+            for (int w = 0; w < kScanWaves; w++) {
+                total = VecT::combine(total, waveTotals[w]);
+            }
+            aggregates[gridDim.x] = total;
+        }
+    } else {
+        prefix = aggregates[blockIdx.x];
+    }
     for (uint32_t w = 0; w < wave; w++) {
         prefix = VecT::combine(prefix, waveTotals[w]);
     }
@@ -210,14 +234,39 @@ inline size_t scanScratchBytes(uint64_t count) {
     return (tiles + 1) * sizeof(VecT);
 }
 
+template <int ITEMS>
+inline uint32_t scanTiles(uint64_t count) {
+    return std::max<uint32_t>(1, ceilDiv(count, uint64_t(kScanThreads) * ITEMS));
+}
+
+// The two halves of scanPipeline, for callers that need the total before they consume: few tiles
+// (at most kScanThreads) leave their own aggregates, whose total is for the caller to sum; more are
+// scanned, the total past them.
+template <class VecT, int ITEMS, class Producer>
+inline void scanReduce(hipStream_t stream, uint32_t count, Producer produce, VecT* aggregates) {
+    const uint32_t tiles = scanTiles<ITEMS>(count);
+    scanReduceKernel<VecT, ITEMS><<<tiles, kScanThreads, 0, stream>>>(produce, count, aggregates);
+    if (tiles > kScanThreads) {
+        scanAggregatesKernel<VecT><<<1, kScanThreads, 0, stream>>>(aggregates, tiles);
+    }
+}
+
+template <class VecT, int ITEMS, class Producer, class Consumer>
+inline void scanDownsweep(hipStream_t stream, uint32_t count, Producer produce, Consumer consume, VecT* aggregates) {
+    const uint32_t tiles = scanTiles<ITEMS>(count);
+    if (tiles > kScanThreads) {
+        scanDownsweepKernel<VecT, ITEMS, false><<<tiles, kScanThreads, 0, stream>>>(produce, consume, count, aggregates);
+    } else {
+        scanDownsweepKernel<VecT, ITEMS, true><<<tiles, kScanThreads, 0, stream>>>(produce, consume, count, aggregates);
+    }
+}
+
 // Runs produce/consume over [0, count). aggregates holds scanScratchBytes; afterwards
 // aggregates[tiles] is the total.
 template <class VecT, int ITEMS, class Producer, class Consumer>
 inline void scanPipeline(hipStream_t stream, uint32_t count, Producer produce, Consumer consume, VecT* aggregates) {
-    const uint32_t tiles = std::max<uint32_t>(1, ceilDiv(count, uint64_t(kScanThreads) * ITEMS));
-    scanReduceKernel<VecT, ITEMS><<<tiles, kScanThreads, 0, stream>>>(produce, count, aggregates);
-    scanAggregatesKernel<VecT><<<1, kScanThreads, 0, stream>>>(aggregates, tiles);
-    scanDownsweepKernel<VecT, ITEMS><<<tiles, kScanThreads, 0, stream>>>(produce, consume, count, aggregates);
+    scanReduce<VecT, ITEMS>(stream, count, produce, aggregates);
+    scanDownsweep<VecT, ITEMS>(stream, count, produce, consume, aggregates);
 }
 
 using Sum1 = Vec<1, 0u>;
