@@ -145,7 +145,8 @@ __global__ __launch_bounds__(256) void bytePresenceKernel(const uint4* __restric
     for (int offset = 8; offset < kWave; offset *= 2) {
         mask |= __shfl_xor(mask, offset);
     }
-    if (threadIdx.x % kWave < 8 && mask) {
+    // Most waves find their bytes there already: 64K atomics on the same eight words took 90 us.
+    if (threadIdx.x % kWave < 8 && (mask & ~__builtin_nontemporal_load(&present[x]))) {
         atomicOr(&present[x], mask);
     }
 }
@@ -518,7 +519,7 @@ constexpr size_t kSliceRowWords = 1024;
 constexpr uint64_t kSliceRows = uint64_t(1) << 24;
 constexpr int64_t kMemoryReserve = int64_t(256) << 20;
 constexpr size_t kTextPadding = 64;
-constexpr size_t kFreeBudget = size_t(256) << 20;
+constexpr size_t kFreeBudget = size_t(1) << 30;
 
 bool gTablesReady[2] = {false, false};
 
@@ -752,7 +753,7 @@ class Pipeline {
     int alphabet(CodeTable& codes, int& sigma, int& charBits, uint32_t* byteCounts) {
         if (!m_job.alphabetKnown) {
             fillWords(byteCounts, 8, 0);
-            bytePresenceKernel<Texts><<<std::min<unsigned>(blocksFor((m_job.span + 15) / 16), 2048), 256, 0, m_stream>>>(
+            bytePresenceKernel<Texts><<<std::min<unsigned>(blocksFor((m_job.span + 15) / 16), 1024), 256, 0, m_stream>>>(
                 reinterpret_cast<const uint4*>(m_job.text), m_job.span, m_texts, byteCounts);
             SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, byteCounts, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
             SADCS_HIP(hipStreamSynchronize(m_stream));
@@ -1373,13 +1374,18 @@ class Pipeline {
         const uint64_t fixedBytes = 16 * Arena::kAlign + (2ull * maxRoundBuckets + 4 + static_cast<uint64_t>(maxRoundBuckets) * bins) * sizeof(uint32_t) +
                                     (bins > 1 ? 2 * sizeof(uint32_t) * static_cast<uint64_t>(maxRoundBuckets) * bins : 0);
         const uint64_t available = budget > m_arena.live() + fixedBytes ? budget - m_arena.live() - fixedBytes : 0;
-        // A large text's second level takes a quarter of a round at a time (fewer rounds, each of which
-        // reads the text again) in tiles of several blocks; a small one's launches would be too short.
+        // A large text's second level takes a quarter or an eighth of a round at a time (fewer rounds, each
+        // of which reads the text again) in tiles of several blocks; a small one's launches would be too short.
         const bool largeText = N >= (uint64_t(1) << 26);
         const uint32_t tileRecords = largeText ? 4 * kPrefixBlock : kPrefixBlock;
-        const uint32_t binGroups = N >= (uint64_t(1) << 29) ? 8 : largeText ? 4 : 1;
-        const double perRecord = sizeof(PrefixRecord) * 1.0 + (bins > 1 ? (sizeof(PrefixRecord) + 2.0 * sizeof(uint32_t) * bins / tileRecords) / binGroups : 0.0);
-        const uint64_t capacity = std::min<uint64_t>(N, static_cast<uint64_t>(available / perRecord));
+        auto perRecord = [&](uint32_t groups) {
+            return sizeof(PrefixRecord) * 1.0 + (bins > 1 ? (sizeof(PrefixRecord) + 2.0 * sizeof(uint32_t) * bins / tileRecords) / groups : 0.0);
+        };
+        uint32_t binGroups = N >= (uint64_t(1) << 29) ? 8 : largeText ? 4 : 1;
+        if (!largeText && available / perRecord(1) < N && available / perRecord(2) >= N) {
+            binGroups = 2;  // one round all the same
+        }
+        const uint64_t capacity = std::min<uint64_t>(N, static_cast<uint64_t>(available / perRecord(binGroups)));
         struct Round {
             uint32_t first, count, rows;
         };
@@ -2710,7 +2716,17 @@ int downloadSlices(sadcs_ctx& ctx, const OutputSlices& o) {
     return SADCS_OK;
 }
 
-int createContext(size_t arenaBytes, const Params& params, int32_t capacity, sadcs_ctx*& out) {
+// Beyond its plan a context for up to this many bytes of text takes kRoomyBytes more a byte, if that is
+// a small part of the free memory: the prefix sort then holds all records at once instead of reading
+// the text once a round (8 MiB: one round instead of five).
+constexpr int64_t kRoomyText = int64_t(48) << 20;
+constexpr int64_t kRoomyBytes = 22;
+
+size_t roomyBytes(int64_t text) {
+    return text <= kRoomyText ? static_cast<size_t>(text * kRoomyBytes) : 0;
+}
+
+int createContext(size_t arenaBytes, const Params& params, int32_t capacity, sadcs_ctx*& out, size_t optional = 0) {
     out = nullptr;
     sadcs_device device;
     SADCS_TRY(queryDevice(device));
@@ -2732,7 +2748,15 @@ int createContext(size_t arenaBytes, const Params& params, int32_t capacity, sad
     SADCS_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     SADCS_HIP(hipDeviceGetAttribute(&ctx->sms, hipDeviceAttributeMultiprocessorCount, 0));
     ctx->arenaBytes = std::max<size_t>(arenaBytes, Arena::kAlign);
-    {
+    if (optional > 0 && static_cast<int64_t>(arenaBytes + optional) + kMemoryReserve <= device.free_bytes / 4) {
+        if (hipMalloc(&ctx->arenaBase, ctx->arenaBytes + optional) == hipSuccess) {
+            ctx->arenaBytes += optional;
+        } else {
+            (void)hipGetLastError();
+            ctx->arenaBase = nullptr;
+        }
+    }
+    if (!ctx->arenaBase) {
         const hipError_t e = hipMalloc(&ctx->arenaBase, ctx->arenaBytes);
         if (e != hipSuccess) {
             setError("hipMalloc(%zu): %s", ctx->arenaBytes, hipGetErrorString(e));
@@ -3384,7 +3408,7 @@ int sadcs_hip_ctx_create_batch(const int64_t* lengths, int32_t count, const sadc
         setError("planning the device memory failed");
         return SADCS_FAILED;
     }
-    return createContext(plan, p, static_cast<int32_t>(longest), *context);
+    return createContext(plan, p, static_cast<int32_t>(longest), *context, p.tiles ? 0 : roomyBytes(total));
 }
 
 int sadcs_hip_ctx_create(int32_t capacity, const sadcs_params* params, sadcs_ctx** context) {
@@ -3408,7 +3432,7 @@ int sadcs_hip_ctx_create(int32_t capacity, const sadcs_params* params, sadcs_ctx
         setError("planning the device memory failed");
         return SADCS_FAILED;
     }
-    return createContext(plan, p, std::max(capacity, 0), *context);
+    return createContext(plan, p, std::max(capacity, 0), *context, p.tiles ? 0 : roomyBytes(std::max(capacity, 0)));
 }
 
 void sadcs_hip_ctx_destroy(sadcs_ctx* context) {
