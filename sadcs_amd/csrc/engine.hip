@@ -978,7 +978,7 @@ class Pipeline {
                 times.doublingRounds += static_cast<int>(m_ctx.hostWords[1]);
                 if (m_ctx.hostWords[2] != 0) {
                     setError("sample ranking: groups left after doubling past the longest text (internal error)");
-                                        return SADCS_FAILED;
+                    return SADCS_FAILED;
                 }
                 break;
             }
@@ -1001,7 +1001,7 @@ class Pipeline {
                 const uint64_t h = depth / V * V;
                 if (h >= m_job.maxLength) {
                     setError("sample ranking: groups left at depth %llu (internal error)", static_cast<unsigned long long>(depth));
-                                        return SADCS_FAILED;
+                    return SADCS_FAILED;
                 }
                 spec.doubling = true;
                 spec.offset = static_cast<uint32_t>(h);
@@ -1697,7 +1697,7 @@ class Pipeline {
                 releaseTaken();
                 return SADCS_OK;
             }
-                        const int rankBits = bitWidth(m_samples);
+            const int rankBits = bitWidth(m_samples);
             const int groupBits = bitWidth(large / kTieGroupMax);
             const int classBits = bitWidth(kClasses);
             fillWords(errors, 1, 0);

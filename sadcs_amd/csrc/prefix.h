@@ -848,6 +848,7 @@ constexpr int kLeafLane = 8;                             // records a lane sorts
 constexpr uint32_t kLeafChunk = kWave * kLeafLane;       // records a wave sorts in registers
 constexpr int kLeafIndexBits = 12;                       // of a record's index in its leaf
 constexpr uint32_t kLeafIndexMask = (1u << kLeafIndexBits) - 1;
+constexpr uint32_t kLeafLastValues = 16;                  // of a key's last four bits
 
 // Lane l's value of lane l ^ kStride.
 template <int kStride>
@@ -906,6 +907,10 @@ __device__ __forceinline__ void bitonicSort(uint64_t (&v)[kLeafLane], uint32_t l
         bitonicSort<kRun / 2>(v, lane);
     }
     bitonicStages<kRun, kRun / 2>(v, lane);
+}
+
+__device__ __forceinline__ uint32_t lastBits(uint64_t key) {
+    return (static_cast<uint32_t>(key) >> 8) & (kLeafLastValues - 1);
 }
 
 // Where value e of a leaf lies in LDS: a lane's eight values are written one after another, and
@@ -970,6 +975,7 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
     __shared__ uint32_t position[kCapacity];
     __shared__ uint8_t before[kCapacity];
     __shared__ uint32_t differLow, differHigh;
+    __shared__ uint32_t lastStart[kLeafLastValues], lastNext[kLeafLastValues];  // truncated leaves
 
     const uint32_t t = threadIdx.x, wave = t / kWave, lane = t % kWave;
     const uint32_t first = leafStart[blockIdx.x] - leafBase;
@@ -994,6 +1000,9 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
     if (t == 0) {
         differLow = 0;
         differHigh = 0;
+    }
+    if (t < kLeafLastValues) {
+        lastNext[t] = 0;
     }
     const uint32_t chunks = (size + kLeafChunk - 1) / kLeafChunk;
     records += first;
@@ -1031,9 +1040,32 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
     __syncthreads();
     const uint64_t differing = static_cast<uint64_t>(differHigh) << 32 | differLow;
     // The bits all keys share at the top; 4 or more leave room for the index. With fewer, the last
-    // four key bits are left out of the values and ordered afterwards.
+    // four key bits are left out of the values: the records are numbered in the order of those bits,
+    // so that the index orders them.
     const int shared = differing ? min(__builtin_clzll(differing), 63) : 63;
     const bool truncated = shared < kLeafIndexBits - 8;
+    if (truncated) {
+#pragma unroll
+        for (int c = 0; c < kPasses; c++) {
+#pragma unroll
+            for (int r = 0; r < kLeafLane; r++) {
+                if ((wave + c * kLeafWaves) * kLeafChunk + r * kWave + lane < size) {
+                    atomicAdd(&lastNext[lastBits(key[c][r])], 1u);
+                }
+            }
+        }
+        __syncthreads();
+        if (t == 0) {
+            uint32_t before16 = 0;
+            for (uint32_t d = 0; d < kLeafLastValues; d++) {
+                const uint32_t count = lastNext[d];
+                lastStart[d] = before16;
+                lastNext[d] = before16;
+                before16 += count;
+            }
+        }
+        __syncthreads();
+    }
 
 #pragma unroll
     for (int c = 0; c < kPasses; c++) {
@@ -1042,7 +1074,13 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
             uint64_t v[kLeafLane];
 #pragma unroll
             for (int r = 0; r < kLeafLane; r++) {
-                const uint32_t x = chunk * kLeafChunk + r * kWave + lane;
+                uint32_t x = chunk * kLeafChunk + r * kWave + lane;
+                if (truncated && x < size) {
+                    const uint32_t from = x;
+                    x = atomicAdd(&lastNext[lastBits(key[c][r])], 1u);
+                    position[x] = records[from].position;
+                    before[x] = static_cast<uint8_t>(key[c][r]);
+                }
                 v[r] = x < size ? ((keyPart(key[c][r]) << shared) & ~static_cast<uint64_t>(kLeafIndexMask)) | x : ~uint64_t(0);
             }
             if (differing) {
@@ -1068,36 +1106,6 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
                 mergeLeafRuns<kLeafLane * kPasses>(values, chunks * kLeafChunk, run);
             }
         }
-        if (truncated) {
-            // Order each run of equal values by the four bits left out: a record's place is the number
-            // of its run's records before it.
-            uint64_t moved[kCapacity / kLeafThreads];
-            uint32_t target[kCapacity / kLeafThreads];
-#pragma unroll
-            for (uint32_t k = 0; k < kCapacity / kLeafThreads; k++) {
-                const uint32_t x = k * kLeafThreads + t;
-                target[k] = x;
-                if (x < size) {
-                    const uint64_t v = values[leafSlot(x)];
-                    moved[k] = v;
-                    const uint32_t own = records[v & kLeafIndexMask].low & 0xF00u;
-                    for (uint32_t y = x; y-- > 0 && values[leafSlot(y)] >> kLeafIndexBits == v >> kLeafIndexBits;) {
-                        target[k] -= (records[values[leafSlot(y)] & kLeafIndexMask].low & 0xF00u) > own ? 1 : 0;
-                    }
-                    for (uint32_t y = x + 1; y < size && values[leafSlot(y)] >> kLeafIndexBits == v >> kLeafIndexBits; y++) {
-                        target[k] += (records[values[leafSlot(y)] & kLeafIndexMask].low & 0xF00u) < own ? 1 : 0;
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (uint32_t k = 0; k < kCapacity / kLeafThreads; k++) {
-                if (k * kLeafThreads + t < size) {
-                    values[leafSlot(target[k])] = moved[k];
-                }
-            }
-            __syncthreads();
-        }
     }
 
     const uint64_t top = differing ? (shared ? reference & ~(~uint64_t(0) >> shared) : 0) : keyPart(reference);
@@ -1109,9 +1117,13 @@ __global__ __launch_bounds__(kLeafThreads) void sortLeavesKernel(const PrefixRec
         bool tied = valid && x > 0 && previous >> kLeafIndexBits == v >> kLeafIndexBits;
         uint64_t key = differing ? top | (v & ~static_cast<uint64_t>(kLeafIndexMask)) >> shared : top;
         if (truncated) {
-            const uint32_t own = records[index].low & 0xF00u;
-            key |= own;
-            tied = tied && (records[previous & kLeafIndexMask].low & 0xF00u) == own;
+            uint32_t last = 0;
+#pragma unroll
+            for (uint32_t step = kLeafLastValues / 2; step > 0; step /= 2) {
+                last += lastStart[last + step] <= index ? step : 0;
+            }
+            key |= static_cast<uint64_t>(last) << 8;
+            tied = tied && (previous & kLeafIndexMask) >= lastStart[last];
         }
         if (valid) {
             emitRow(out, rowBase + first + x, key | before[index], position[index], tied);

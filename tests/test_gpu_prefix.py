@@ -74,6 +74,22 @@ def test_prefix_large(gpu, kind, n, cover):
     check_device(gpu, text_of(kind, n), cover)
 
 
+@pytest.mark.parametrize("run", [700, 2047, 3900])
+def test_prefix_leaf_spanning_first_bits(gpu, run):
+    # Letters 3 and 4 of 8: keys 011... and 100... share a leaf, so its values hold no last four bits,
+    # and a run's keys differ in those alone.
+    rng = np.random.default_rng(run)
+    text = rng.integers(0, 8, 20_000 + run, dtype=np.uint8)
+    text[5000:5000 + run] = 3
+    text[15000:15000 + run // 2] = 4
+    for at in range(5000 + 16, 5000 + run, 400):  # breaks: a key's 18 letters end before, at and behind
+        text[at] = rng.integers(0, 8)
+    sa, bwt, primary = check_device(gpu, text)
+    want = oracle.suffix_array(text.tobytes())
+    assert np.array_equal(sa, want)
+    assert (bwt, primary) == oracle.bwt_from_sa(text.tobytes(), want)
+
+
 def test_prefix_batches(gpu):
     from sadcs_amd import workloads
     rng = np.random.default_rng(5)
