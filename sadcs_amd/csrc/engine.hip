@@ -2600,6 +2600,43 @@ int upload(sadcs_ctx& ctx, void* device, const void* host, size_t bytes, bool& p
     return SADCS_OK;
 }
 
+// A batch's texts to their places (device[0, span), zeros between them), gathered in the pinned
+// chunks: one DMA a piece instead of one a text, each of which costs about 14 us whatever its size
+// (680 texts of up to 61,176 bytes: 15.4 -> 5.3 ms for the whole call).
+template <class TextOf>
+int uploadGathered(sadcs_ctx& ctx, uint8_t* device, const std::vector<Segment>& segments, size_t span, TextOf textOf) {
+    const size_t piece = stagingPiece(span);
+    std::vector<HostCopier::Piece> copies;
+    size_t i = 0;
+    for (size_t k = 0, offset = 0; offset < span; k++, offset += piece) {
+        const size_t end = std::min(offset + piece, span);
+        const int b = static_cast<int>(k & 1);
+        SADCS_HIP(hipEventSynchronize(ctx.stagingDone[b]));
+        uint8_t* staged = ctx.staging[b];
+        copies.clear();
+        size_t at = offset;  // staged up to here
+        while (at < end) {
+            const size_t textStart = i < segments.size() ? segments[i].start : span;
+            const size_t textEnd = i < segments.size() ? segments[i].end : span;
+            if (at < textStart) {
+                const size_t to = std::min(textStart, end);
+                memset(staged + (at - offset), 0, to - at);
+                at = to;
+            } else if (at < textEnd) {
+                const size_t to = std::min(textEnd, end);
+                copies.push_back({staged + (at - offset), textOf(i) + (at - textStart), to - at});
+                at = to;
+            } else {
+                i++;
+            }
+        }
+        HostCopier::instance().copyPieces(copies.data(), copies.size());
+        SADCS_HIP(hipMemcpyAsync(device + offset, staged, end - offset, hipMemcpyHostToDevice, ctx.stream));
+        SADCS_HIP(hipEventRecord(ctx.stagingDone[b], ctx.stream));
+    }
+    return SADCS_OK;
+}
+
 // Device to host after the stream's earlier work; returns with the data on the host.
 int download(sadcs_ctx& ctx, void* host, const void* device, size_t bytes) {
     if (bytes == 0) {
@@ -2906,15 +2943,23 @@ int buildWith(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, Text
     bool pinned = false;
     if (!deviceCall) {
         const auto start = std::chrono::steady_clock::now();
-        SADCS_HIP(hipMemsetAsync(in.text, 0, static_cast<size_t>(layout.span) + kTextPadding + 8, ctx.stream));
+        const size_t span = layout.span, texts = layout.segments.size();
+        std::vector<size_t> offsets(batch && !rq.hostTexts ? texts : 0);
+        for (size_t i = 1; i < offsets.size(); i++) {
+            offsets[i] = offsets[i - 1] + (layout.segments[i - 1].end - layout.segments[i - 1].start);
+        }
+        auto textOf = [&](size_t i) { return rq.hostTexts ? rq.hostTexts[i] : rq.hostText + offsets[i]; };
+        const bool gather = batch && ctx.staging[0] && ctx.staging[1] && !isPinned(textOf(0));  // pinned texts need no staging
+        const size_t cleared = batch && !gather ? 0 : span & ~size_t(255);
+        SADCS_HIP(hipMemsetAsync(in.text + cleared, 0, span - cleared + kTextPadding + 8, ctx.stream));
         if (!batch) {
-            SADCS_TRY(upload(ctx, in.text, rq.hostText, layout.span, pinned));
+            SADCS_TRY(upload(ctx, in.text, rq.hostText, span, pinned));
+        } else if (gather) {
+            pinned = true;
+            SADCS_TRY(uploadGathered(ctx, in.text, layout.segments, span, textOf));
         } else {
-            const uint8_t* src = rq.hostText;
-            for (size_t i = 0; i < layout.segments.size(); i++) {
-                const size_t n = layout.segments[i].end - layout.segments[i].start;
-                SADCS_TRY(upload(ctx, in.text + layout.segments[i].start, rq.hostTexts ? rq.hostTexts[i] : src, n, pinned));
-                src += n;
+            for (size_t i = 0; i < texts; i++) {
+                SADCS_TRY(upload(ctx, in.text + layout.segments[i].start, textOf(i), layout.segments[i].end - layout.segments[i].start, pinned));
             }
         }
         SADCS_HIP(hipStreamSynchronize(ctx.stream));

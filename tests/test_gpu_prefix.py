@@ -115,3 +115,14 @@ def test_prefix_batches(gpu):
             result = gpu.gpu_check_device(d_texts.ptr + int(offsets[i]), t.size, d_sa.ptr + 4 * at, d_bwt.ptr + at, int(primaries[i]))
             assert result == (0, -1), f"text {i} of {t.size} bytes"
             at += t.size
+
+
+def test_host_batch_gathered_in_pieces(gpu):
+    # Texts that end before, at and past the 2 MiB pieces of the upload, and one over three of them.
+    from sadcs_amd import workloads
+    mib = 1 << 20
+    lengths = [2 * mib - 100, 2 * mib, 300, 2 * mib - 512 + 1, 70_000, 1, 4 * mib + 255, 20_000]
+    texts = [workloads.protein(n, seed=n & 1023) for n in lengths]
+    for text, (sa, bwt, primary) in zip(texts, gpu.gpu_batch_build(texts, True, True)):
+        want = gpu.gpu_build(text, True, True)
+        assert np.array_equal(sa, want[0]) and (bwt, primary) == want[1:]
