@@ -555,6 +555,12 @@ uint64_t classSizeOf(uint64_t n, int d) {
 // radix passes.
 constexpr uint64_t kGroupRankMeanMax = 8;
 
+// Lists up to this long are scanned while the host does not know yet whether all of it is sorted.
+constexpr uint32_t kGuessMax = 1 << 20;
+
+// Lists up to this long are doubled with every id that fits the key.
+constexpr uint32_t kWideKeysMax = 1 << 18;
+
 // The first ranking pass of a large sample leaves its resolved rank stores to
 // scatterResolvedRanksKernel, in launches over consecutive rank ranges of at most this many bytes
 // (what the 256 MB memory-side cache holds: at 1 GiB, 4 launches measured 1.2 ms faster than 8,
@@ -950,6 +956,7 @@ class Pipeline {
         int listBuffer = state.listBuffer;  // where the list's t and ordinals are (values[x], keys[x] as words)
         int gcur = state.groupBuffer;
         const int rankBits = bitWidth(m_samples);
+        uint32_t largeBefore = 0;  // elements of large groups in the last pass sorted within groups
 
         while (u > 0) {
             if (!first && u <= kTailMax) {
@@ -966,13 +973,12 @@ class Pipeline {
                 tp.groupIds = groupIds[gcur];
                 tp.u = u;
                 tp.groups = groups;
-                tp.status = counts;
+                tp.status = m_ctx.hostWords;  // pinned: the host reads it where the kernel writes it
                 const size_t tailShared = rankTailSharedBytes();
                 SADCS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rankTailKernel<V, Texts>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               static_cast<int>(tailShared)));
                 rankTailKernel<V, Texts><<<1, kTailThreads, tailShared, m_stream>>>(tp, m_texts);
                 SADCS_HIP(hipGetLastError());
-                SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, counts, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
                 SADCS_HIP(hipStreamSynchronize(m_stream));
                 times.characterPasses += static_cast<int>(m_ctx.hostWords[0]);
                 times.doublingRounds += static_cast<int>(m_ctx.hostWords[1]);
@@ -1005,7 +1011,12 @@ class Pipeline {
                 }
                 spec.doubling = true;
                 spec.offset = static_cast<uint32_t>(h);
-                spec.subkeyBits = rankBits;
+                // Where the passes are launches and waits, or groups are sorted apart whatever the
+                // key's width, as many ids as fit; else each would cost digit passes over the list.
+                const bool wide = u <= kWideKeysMax || u <= kGroupRankMeanMax * static_cast<uint64_t>(groups);
+                spec.ids = wide ? std::max(1, (ordinalBits > 0 ? 63 - ordinalBits : 64) / rankBits) : 1;
+                spec.idBits = rankBits;
+                spec.subkeyBits = spec.ids * rankBits;
             }
 
             const int y = 1 - listBuffer;
@@ -1014,72 +1025,85 @@ class Pipeline {
             const bool identity = first && !kBatch && u > 1;
             uint32_t* valuesOut = identity ? nullptr : values[y];
             uint8_t* digitsOut = first ? digits : nullptr;
+            uint32_t* large = counts;  // elements of groups too large to sort within
             if (charBits == 9 && !spec.doubling) {
                 makePassKeysKernel<V, Texts, true><<<blocksFor(u), 256, 0, m_stream>>>(
-                    rp, m_texts, spec, codes, first, values[listBuffer], reinterpret_cast<const uint32_t*>(keys[listBuffer]), u, keys[y], valuesOut, digitsOut);
+                    rp, m_texts, spec, codes, first, values[listBuffer], reinterpret_cast<const uint32_t*>(keys[listBuffer]), u, keys[y], valuesOut, digitsOut, large);
             } else {
                 makePassKeysKernel<V, Texts, false><<<blocksFor(u), 256, 0, m_stream>>>(
-                    rp, m_texts, spec, codes, first, values[listBuffer], reinterpret_cast<const uint32_t*>(keys[listBuffer]), u, keys[y], valuesOut, digitsOut);
+                    rp, m_texts, spec, codes, first, values[listBuffer], reinterpret_cast<const uint32_t*>(keys[listBuffer]), u, keys[y], valuesOut, digitsOut, large);
             }
             // After the first pass the unresolved groups are mostly pairs: sort within groups. The
             // few elements of groups too large for that (long runs) are sorted apart; when they are
             // many, or the groups are large on average (the scans would cost more than the radix
             // passes), the pass is sorted by radix.
-            bool sorted = false;
+            bool sorted = false, guessed = false;
+            uint32_t largeNow = 0;
             if (!first && ordinalBits > 0 && spec.subkeyBits < 64 && u <= kGroupRankMeanMax * static_cast<uint64_t>(groups)) {
-                SADCS_HIP(hipMemsetAsync(counts + 2, 0, sizeof(uint32_t), m_stream));
-                groupRankSortKernel<<<blocksFor(u), 256, 0, m_stream>>>(keys[y], values[y], u, spec.subkeyBits, keys[1 - y], values[1 - y], digits, counts + 2);
-                SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords + 2, counts + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+                groupRankSortKernel<<<blocksFor(u), 256, 0, m_stream>>>(keys[y], values[y], u, spec.subkeyBits, keys[1 - y], values[1 - y], digits, large);
+                // A short list is scanned without waiting for the count, unless the last pass had
+                // large groups: the wait would cost more than a scan in vain.
+                guessed = largeBefore == 0 && u <= kGuessMax;
+                if (!guessed) {
+                    SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords + 2, large, sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+                    SADCS_HIP(hipStreamSynchronize(m_stream));
+                    largeNow = m_ctx.hostWords[2];
+                    sorted = largeNow == 0;
+                }
+            }
+            auto mark = [&](int c, const uint32_t* unsorted) -> int {
+                MarkState ms{};
+                ms.keys = keys[c];
+                ms.values = values[c];
+                ms.u = u;
+                ms.subkeyBits = spec.subkeyBits;
+                ms.groupIds = groupIds[gcur];
+                ms.ranks = m_ranks;
+                ms.sortedSample = rp.sortedSample;
+                ms.nextT = values[1 - c];
+                ms.nextOrdinal = reinterpret_cast<uint32_t*>(keys[1 - c]);
+                ms.nextGroupIds = groupIds[1 - gcur];
+                ms.counts = m_ctx.hostWords;
+                ms.large = unsorted;
+                ms.samples = M;
+                ms.deferResolved = first && u >= kDeferredRankMin;
+                scanPipeline<MarkVec, kMarkItems>(m_stream, u, MarkProducer{ms}, MarkConsumer<V>{ms}, markAggregates);
+                SADCS_HIP(hipGetLastError());
+                if (ms.deferResolved) {
+                    const uint32_t rankCount = static_cast<uint32_t>(Cover::pack(m_job.span));
+                    const uint64_t rounds = std::max<uint64_t>(1, (uint64_t(rankCount) * sizeof(uint32_t) + kDeferredRankWindow - 1) / kDeferredRankWindow);
+                    const uint32_t step = static_cast<uint32_t>((rankCount + rounds - 1) / rounds);
+                    const unsigned grid = std::min<unsigned>(blocksFor(M), 8192);
+                    for (uint32_t lo = 0; lo < rankCount; lo += step) {
+                        scatterResolvedRanksKernel<V><<<grid, 256, 0, m_stream>>>(m_lists[0], M, lo, std::min(rankCount, lo + step), m_ranks);
+                    }
+                    SADCS_HIP(hipGetLastError());
+                }
                 SADCS_HIP(hipStreamSynchronize(m_stream));
-                const uint32_t large = m_ctx.hostWords[2];
-                if (large == 0) {
-                    sorted = true;
-                } else if (large <= u / 4) {
-                    SADCS_TRY(sortLargeGroups(keys, values, y, u, large, ordinalBits + spec.subkeyBits, digits, hist, sortAggregates,
+                return SADCS_OK;
+            };
+            int c = 1 - y;
+            if (guessed) {
+                SADCS_TRY(mark(c, large));
+                largeNow = m_ctx.hostWords[2];
+            }
+            if (!guessed || largeNow != 0) {
+                if (!sorted && largeNow != 0 && largeNow <= u / 4) {
+                    SADCS_TRY(sortLargeGroups(keys, values, y, u, largeNow, ordinalBits + spec.subkeyBits, digits, hist, sortAggregates,
                                               reinterpret_cast<Sum1*>(markAggregates), sorted));
                 }
-                if (sorted) {
-                    sb.current = 1 - y;
+                if (!sorted) {
+                    sb.current = y;
+                    sb.identityValues = identity;
+                    sb.digitsReady = first;
+                    radixSort<uint64_t>(m_stream, sb, u, 0, ordinalBits + spec.subkeyBits);
+                    sb.identityValues = false;
+                    sb.digitsReady = false;
+                    c = sb.current;
                 }
+                SADCS_TRY(mark(c, nullptr));
             }
-            if (!sorted) {
-                sb.current = y;
-                sb.identityValues = identity;
-                sb.digitsReady = first;
-                radixSort<uint64_t>(m_stream, sb, u, 0, ordinalBits + spec.subkeyBits);
-                sb.identityValues = false;
-                sb.digitsReady = false;
-            }
-            const int c = sb.current;
-
-            MarkState ms{};
-            ms.keys = keys[c];
-            ms.values = values[c];
-            ms.u = u;
-            ms.subkeyBits = spec.subkeyBits;
-            ms.groupIds = groupIds[gcur];
-            ms.ranks = m_ranks;
-            ms.sortedSample = rp.sortedSample;
-            ms.nextT = values[1 - c];
-            ms.nextOrdinal = reinterpret_cast<uint32_t*>(keys[1 - c]);
-            ms.nextGroupIds = groupIds[1 - gcur];
-            ms.counts = counts;
-            ms.samples = M;
-            ms.deferResolved = first && u >= kDeferredRankMin;
-            scanPipeline<MarkVec, kMarkItems>(m_stream, u, MarkProducer{ms}, MarkConsumer<V>{ms}, markAggregates);
-            SADCS_HIP(hipGetLastError());
-            if (ms.deferResolved) {
-                const uint32_t rankCount = static_cast<uint32_t>(Cover::pack(m_job.span));
-                const uint64_t rounds = std::max<uint64_t>(1, (uint64_t(rankCount) * sizeof(uint32_t) + kDeferredRankWindow - 1) / kDeferredRankWindow);
-                const uint32_t step = static_cast<uint32_t>((rankCount + rounds - 1) / rounds);
-                const unsigned grid = std::min<unsigned>(blocksFor(M), 8192);
-                for (uint32_t lo = 0; lo < rankCount; lo += step) {
-                    scatterResolvedRanksKernel<V><<<grid, 256, 0, m_stream>>>(m_lists[0], M, lo, std::min(rankCount, lo + step), m_ranks);
-                }
-                SADCS_HIP(hipGetLastError());
-            }
-            SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, counts, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
-            SADCS_HIP(hipStreamSynchronize(m_stream));
+            largeBefore = largeNow;
 
             u = m_ctx.hostWords[0];
             groups = m_ctx.hostWords[1];
@@ -1087,7 +1111,7 @@ class Pipeline {
             listBuffer = 1 - c;
             first = false;
             if (spec.doubling) {
-                depth += spec.offset;
+                depth += static_cast<uint64_t>(spec.offset) * spec.ids;
                 times.doublingRounds++;
             } else {
                 depth += static_cast<uint64_t>(spec.chars);
