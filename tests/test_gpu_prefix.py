@@ -126,3 +126,14 @@ def test_host_batch_gathered_in_pieces(gpu):
     for text, (sa, bwt, primary) in zip(texts, gpu.gpu_batch_build(texts, True, True)):
         want = gpu.gpu_build(text, True, True)
         assert np.array_equal(sa, want[0]) and (bwt, primary) == want[1:]
+
+
+@pytest.mark.parametrize("n", [4096 - 7, 4096, 4096 + 9, 8192 + 1, 12_288 - 5, 33_000, 65_536 + 40, 300_007, 2_097_152 + 16, 2_200_000])
+def test_sample_sorted_by_merges(gpu, n):
+    # The ranking sorts about n / 4 sample keys: under, at and over the chunks that a workgroup sorts,
+    # odd numbers of runs, and over the length from which digit passes take them. The suffix array that
+    # the ranks imply comes from another path.
+    from sadcs_amd import workloads
+    for text in (workloads.dna_like(n, seed=5), workloads.periodic(n, seed=6)):
+        sa, _, _ = check_device(gpu, text)
+        assert np.array_equal(gpu.gpu_rank_sample(text), oracle.sample_ranks_from_sa(sa, 32))
