@@ -137,3 +137,18 @@ def test_sample_sorted_by_merges(gpu, n):
     for text in (workloads.dna_like(n, seed=5), workloads.periodic(n, seed=6)):
         sa, _, _ = check_device(gpu, text)
         assert np.array_equal(gpu.gpu_rank_sample(text), oracle.sample_ranks_from_sa(sa, 32))
+
+
+@pytest.mark.parametrize("n", [16_385, 118_796, 1_048_577, 5_000_011])
+def test_cover_128_by_cover_32(gpu, n):
+    # Texts that the prefix sort leaves to the tile merge: a context of cover 128 with room for it takes
+    # cover 32, one with merge parameters its own.
+    for kind in ("periodic", "zeros"):
+        text = text_of(kind, n)
+        d_text = gpu.DeviceBuffer.from_host(text, extra=64)
+        d_sa, d_bwt = gpu.DeviceBuffer(4 * n), gpu.DeviceBuffer(n)
+        with gpu.GpuContext(n, cover=128, tile_splitters=8) as ctx:
+            primary = gpu.gpu_build_device(ctx, d_text.ptr, n, d_sa.ptr, d_bwt.ptr)
+        assert gpu.gpu_check_device(d_text.ptr, n, d_sa.ptr, d_bwt.ptr, primary) == (0, -1)
+        sa, bwt, got = check_device(gpu, text, cover=128)
+        assert np.array_equal(sa, d_sa.to_host(np.int32)) and bwt == d_bwt.to_host(np.uint8).tobytes() and got == primary
