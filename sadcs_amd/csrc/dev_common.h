@@ -223,4 +223,25 @@ struct TextBatch {
     static constexpr bool kBatch = true;
 };
 
+// Lane l's value of lane l ^ kStride.
+template <int kStride>
+__device__ __forceinline__ uint32_t laneXor(uint32_t x) {
+    if constexpr (kStride == 1) {
+        return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0xB1, 0xF, 0xF, true));  // quad_perm 1 0 3 2
+    } else if constexpr (kStride == 2) {
+        return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x4E, 0xF, 0xF, true));  // quad_perm 2 3 0 1
+    } else if constexpr (kStride == 8) {
+        return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), 0x128, 0xF, 0xF, true));  // row_ror 8
+    } else if constexpr (kStride == 4 || kStride == 16) {
+        return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(x), kStride << 10 | 0x1F));  // xor within 32 lanes
+    } else {
+        return __shfl_xor(x, kStride);
+    }
+}
+
+template <int kStride>
+__device__ __forceinline__ uint64_t laneXor64(uint64_t x) {
+    return static_cast<uint64_t>(laneXor<kStride>(static_cast<uint32_t>(x >> 32))) << 32 | laneXor<kStride>(static_cast<uint32_t>(x));
+}
+
 }  // namespace sadcs

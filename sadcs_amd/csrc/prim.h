@@ -705,53 +705,109 @@ inline void radixPassDigits(hipStream_t stream, SortBuffers<K>& b, Source source
 //
 // A digit pass over up to some 100,000 items is three launches of 5 to 10 us each, whatever it moves:
 // eight of them for the 64-bit keys of a few thousand items. Sorting chunks in LDS and merging the
-// runs pairwise takes one launch and one more for each doubling of the run. The chunks are small: a
-// stage of the network waits on LDS and a barrier (55 of them 19 us for 1024 items, 78 of them 53 us
-// for 4096), a launch of the merge on its probes of memory (4.4 us).
+// runs pairwise takes one launch and one more for each doubling of the run. A chunk's waves
+// sort in registers: a bitonic network in LDS waits on LDS and a barrier 55 times (19 us for chunks of
+// 1024 against 10; 53 us for 4096), a launch of the merge on its few probes of memory (4.7 us).
 
-constexpr uint32_t kChunk = 1024;         // items a workgroup sorts in LDS
-constexpr int kChunkThreads = kChunk / 2;
+constexpr int kChunkLane = 4;             // items a lane sorts in registers
+constexpr uint32_t kChunkWave = kWave * kChunkLane;
+constexpr int kChunkThreads = 256;
+constexpr uint32_t kChunk = kChunkThreads * kChunkLane;  // items a workgroup sorts
 constexpr uint32_t kRunTile = 1024;     // outputs of a workgroup of mergeRunsKernel
 constexpr int kRunThreads = 256;
 constexpr int kRunItems = kRunTile / kRunThreads;
 
-// Chunk blockIdx.x stably by the bits from beginBit on: a bitonic network on (key, index).
-template <class K>
-__global__ __launch_bounds__(kChunkThreads) void sortChunksKernel(const K* __restrict__ keys, const uint32_t* __restrict__ values, uint32_t count, int beginBit, K* __restrict__ keysOut, uint32_t* __restrict__ valuesOut) {
-    __shared__ K key[kChunk];
-    __shared__ uint16_t index[kChunk];
-    const uint32_t first = blockIdx.x * kChunk, size = min(kChunk, count - first);
-    uint32_t width = kWave;
-    while (width < size) {
-        width *= 2;
-    }
-    for (uint32_t i = threadIdx.x; i < width; i += kChunkThreads) {
-        key[i] = i < size ? keys[first + i] : ~K(0);
-        index[i] = static_cast<uint16_t>(i);  // those past the end stay there: the last among the largest
-    }
-    __syncthreads();
-    for (uint32_t k = 2; k <= width; k *= 2) {
-        for (uint32_t j = k / 2; j > 0; j /= 2) {
-            for (uint32_t x = threadIdx.x; x < width / 2; x += kChunkThreads) {
-                const uint32_t i = 2 * x - (x & (j - 1)), l = i + j;
-                const K a = key[i], b = key[l];
-                const uint16_t ia = index[i], ib = index[l];
-                const K ka = a >> beginBit, kb = b >> beginBit;
-                const bool greater = ka > kb || (ka == kb && ia > ib);
-                if (greater == ((i & k) == 0)) {
-                    key[i] = b;
-                    key[l] = a;
-                    index[i] = ib;
-                    index[l] = ia;
-                }
+// One phase of the bitonic sort of a wave's kChunkWave items, item lane * kChunkLane + r in key[r],
+// index[r]: sorted runs of kRun / 2, alternately ascending and descending, into runs of kRun.
+template <int kRun, int kStride, class K>
+__device__ __forceinline__ void chunkStages(K (&key)[kChunkLane], uint32_t (&index)[kChunkLane], uint32_t lane) {
+    if constexpr (kStride >= kChunkLane) {
+        constexpr int kLanes = kStride / kChunkLane;
+        const bool keepSmaller = ((lane & kLanes) == 0) == ((lane & (kRun / kChunkLane)) == 0);
+#pragma unroll
+        for (int r = 0; r < kChunkLane; r++) {
+            const K k = static_cast<K>(laneXor64<kLanes>(key[r]));
+            const uint32_t i = laneXor<kLanes>(index[r]);
+            const bool keep = ((key[r] < k) | ((key[r] == k) & (index[r] < i))) == keepSmaller;
+            key[r] = keep ? key[r] : k;
+            index[r] = keep ? index[r] : i;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kChunkLane; r++) {
+            if ((r & kStride) == 0) {
+                const bool ascending = kRun >= kChunkLane ? (lane & (kRun / kChunkLane)) == 0 : (r & kRun) == 0;
+                const K ka = key[r], kb = key[r + kStride];
+                const uint32_t ia = index[r], ib = index[r + kStride];
+                const bool keep = ((ka < kb) | ((ka == kb) & (ia < ib))) == ascending;
+                key[r] = keep ? ka : kb;
+                key[r + kStride] = keep ? kb : ka;
+                index[r] = keep ? ia : ib;
+                index[r + kStride] = keep ? ib : ia;
             }
-            __syncthreads();
         }
     }
-    for (uint32_t i = threadIdx.x; i < size; i += kChunkThreads) {
-        const uint32_t from = first + index[i];
-        keysOut[first + i] = key[i];
-        valuesOut[first + i] = values ? values[from] : from;
+    if constexpr (kStride > 1) {
+        chunkStages<kRun, kStride / 2>(key, index, lane);
+    }
+}
+
+template <int kRun, class K>
+__device__ __forceinline__ void sortChunkWave(K (&key)[kChunkLane], uint32_t (&index)[kChunkLane], uint32_t lane) {
+    if constexpr (kRun > 2) {
+        sortChunkWave<kRun / 2>(key, index, lane);
+    }
+    chunkStages<kRun, kRun / 2>(key, index, lane);
+}
+
+// Chunk blockIdx.x stably by the bits from beginBit on: a wave sorts 256 items in registers, by
+// (key, index), and the waves' runs merge in LDS.
+template <class K>
+__global__ __launch_bounds__(kChunkThreads) void sortChunksKernel(const K* __restrict__ keys, const uint32_t* __restrict__ values, uint32_t count, int beginBit, K* __restrict__ keysOut, uint32_t* __restrict__ valuesOut) {
+    __shared__ K shared[kChunk];
+    __shared__ uint16_t sharedIndex[kChunk];
+    const uint32_t first = blockIdx.x * kChunk, size = min(kChunk, count - first);
+    const uint32_t o = threadIdx.x * kChunkLane, lane = laneId();
+    K key[kChunkLane];
+    uint32_t index[kChunkLane];
+#pragma unroll
+    for (int r = 0; r < kChunkLane; r++) {
+        index[r] = o + r;
+        key[r] = o + r < size ? keys[first + o + r] >> beginBit : ~K(0);  // past the end: the last of the largest
+    }
+    sortChunkWave<kChunkWave>(key, index, lane);
+    for (uint32_t run = kChunkWave; run < kChunk; run *= 2) {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kChunkLane; r++) {
+            shared[o + r] = key[r];
+            sharedIndex[o + r] = static_cast<uint16_t>(index[r]);
+        }
+        __syncthreads();
+        const uint32_t a = o / (2 * run) * (2 * run), b = a + run, d = o - a;
+        uint32_t lo = d > run ? d - run : 0, hi = min(d, run);
+        while (lo < hi) {
+            const uint32_t m = (lo + hi) / 2;
+            const bool take = shared[a + m] <= shared[b + d - 1 - m];
+            lo = take ? m + 1 : lo;
+            hi = take ? hi : m;
+        }
+        uint32_t x = lo, y = d - lo;
+#pragma unroll
+        for (int r = 0; r < kChunkLane; r++) {
+            const bool take = x < run && (y >= run || shared[a + x] <= shared[b + y]);
+            const uint32_t from = take ? a + x++ : b + y++;
+            key[r] = shared[from];
+            index[r] = sharedIndex[from];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kChunkLane; r++) {
+        if (o + r < size) {
+            const uint32_t from = first + index[r];
+            keysOut[first + o + r] = keys[from];
+            valuesOut[first + o + r] = values ? values[from] : from;
+        }
     }
 }
 
@@ -838,8 +894,8 @@ inline void mergeSort(hipStream_t stream, SortBuffers<K>& b, uint32_t count, int
     }
 }
 
-// Up to here the merges win: half a million 64-bit keys of periodic text 2.20 against 2.31 ms for the
-// whole build, 12,000 of them 0.76 against 1.10 ms; at a million the two are even.
+// Up to here the merges win: half a million 64-bit keys of periodic text 2.08 against 2.31 ms for the
+// whole build, 12,000 of them 0.70 against 1.10 ms; at a million the two are even.
 constexpr uint32_t kMergeSortMax = 1 << 19;
 
 // Stable sort of b.keys[current], b.values[current] (count items) by bits [beginBit, endBit); the bits
