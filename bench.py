@@ -7,11 +7,14 @@ merge, with the text already resident in HBM and both outputs left in HBM (the d
 entry point of the C ABI). value = input bytes per second over the timed steps, in decimal MB/s.
 
 Printed as one JSON line, with:
-  roofline: the dominant kernel (the top-level tile merge) - its algorithmic bytes per launch
-    (54 bytes per element for SA + BWT: list entry 4, record 44, SA 4, BWT 2) over its average
-    duration measured with HIP events on the library's stream, against 8 TB/s of HBM; traffic is
-    the kernel's measured HBM bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a copy
-    of known size, profiles/mergeTilesKernel_c3_1GiB_traffic.md);
+  roofline: the kernels that take most of the step, the rounds that put every suffix in the order
+    of its first characters - their algorithmic bytes (54 bytes per element for SA + BWT: text 1,
+    a 12-byte record written and read by each of two scatters, SA 4, BWT 1) over their duration
+    measured with HIP events on the library's stream, against 8 TB/s of HBM. With --tune-mib the
+    build takes the tile merge instead, and the line is its top-level kernel's: 54 bytes per
+    element (list entry 4, record 44, SA 4, BWT 2), traffic its measured HBM bytes per launch
+    (rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a copy of known size,
+    profiles/mergeTilesKernel_c3_1GiB_traffic.md);
   e2e_hbm_fraction: the whole step's algorithmic bytes (127.94 bytes per input byte for fused
     SA + BWT) over the step time, against 8 TB/s;
   host_call: the same 1 GiB text through the host-memory API (pageable text in, SA and BWT out,
@@ -46,6 +49,8 @@ BYTES_PER_INPUT_BYTE = 127.94   # fused SA + BWT, the reference design's logical
 # Top-level merge, per element: list entry 4 + record (16 characters and a 4-byte rank per sample
 # of its window: 7 for cover 32, 13 for cover 128) + SA 4 + BWT 2.
 MERGE_BYTES_PER_ELEMENT = {32: 54.0, 128: 78.0}
+# The prefix sort's rounds: text 1, 12-byte records written and read twice, SA 4, BWT 1.
+ROUNDS_BYTES_PER_ELEMENT = 54.0
 METRIC = "SA+BWT input MB/s at 1 GiB; batched/served MB/s + p99 vs sequential"
 
 
@@ -184,7 +189,7 @@ def batched_measurement(count, steps, tune=True, cpu_texts=0):
     d_bwt = sadcs_amd.DeviceBuffer(total)
     d_sa2 = sadcs_amd.DeviceBuffer(4 * total)
     d_bwt2 = sadcs_amd.DeviceBuffer(total)
-    # Autotune on the first 256 texts (their own batch layout), then build everything with it.
+    # The tile merge: autotuned on the first 256 texts (their own batch layout).
     tuned = {}
     if tune:
         sub_lengths = lengths[:256]
@@ -403,8 +408,8 @@ def main():
     ap.add_argument("--cover", type=int, default=32)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--cpu-runs", type=int, default=3, help="runs of the CPU reference's SA and BWT (best of)")
-    ap.add_argument("--tune-mib", type=int, default=64,
-                    help="autotune the merge configuration on a prefix of this many MiB before timing (0: defaults)")
+    ap.add_argument("--tune-mib", type=int, default=0,
+                    help="build by the tile merge, its configuration tuned on a prefix of this many MiB (0: the default path)")
     ap.add_argument("--batch-texts", type=int, default=4096, help="texts in the batched measurement (0: skip)")
     ap.add_argument("--serve-requests", type=int, default=300, help="requests per offered rate (0: skip)")
     ap.add_argument("--serve-workers", type=int, default=0, help="server workers (0: the library default)")
@@ -494,7 +499,8 @@ def main():
     step = elapsed / args.steps
     value = n / step / 1e6
     kernel = sum(merge_kernel) / len(merge_kernel)
-    achieved = MERGE_BYTES_PER_ELEMENT[args.cover] * n / kernel
+    per_element = MERGE_BYTES_PER_ELEMENT[args.cover] if tuned else ROUNDS_BYTES_PER_ELEMENT
+    achieved = per_element * n / kernel
     e2e = BYTES_PER_INPUT_BYTE * n / step / HBM_PEAK
 
     # The timed output checked whole on the device: a permutation, neighbours in order (the
@@ -542,11 +548,12 @@ def main():
         "config": {"workload": f"{args.config}: {description}", "n": n, "outputs": "SA int32 + BWT, one merge",
                    "cover": args.cover, "resident": "text in HBM before the timed region, outputs in HBM",
                    "merge_params": tuned or "defaults", "tuning_seconds": round(tune_seconds, 2)},
-        "roofline": {"bound": "hbm", "kernel": "mergeTilesKernel (top level, SA+BWT in place)",
+        "roofline": {"bound": "hbm", "kernel": "mergeTilesKernel (top level, SA+BWT in place)" if tuned else
+                     "rounds of scatterBucketsKernel, scatterBinsKernel, sortLeavesKernel",
                      "achieved": round(achieved / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK, 4),
-                     "traffic": measured_traffic(args.config, n) if args.cover == 32 else None,  # measured at cover 32
-                     "alg_bytes_per_launch": int(MERGE_BYTES_PER_ELEMENT[args.cover] * n), "avg_launch_ms": round(kernel * 1e3, 3)},
+                     "traffic": measured_traffic(args.config, n) if tuned and args.cover == 32 else None,  # measured at cover 32
+                     "alg_bytes_per_launch": int(per_element * n), "avg_launch_ms": round(kernel * 1e3, 3)},
         "e2e_hbm_fraction": round(e2e, 4),
         "phases_ms": {"ranking": round(ranking * 1e3, 2), "classes": round(classes * 1e3, 2), "merge": round(merge * 1e3, 2)},
         "peak_device_bytes_per_input_byte": round(peak_bytes / n, 3),

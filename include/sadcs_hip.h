@@ -57,11 +57,17 @@ typedef struct sadcs_stats {
     double merge_seconds;
     double bwt_seconds;
     double download_seconds;
-    double merge_kernel_seconds; /* HIP-event time of the top-level tile-merge kernel on the context's stream */
-    int64_t merge_kernel_elements; /* elements that kernel merged (the whole text) */
+    double merge_kernel_seconds; /* HIP-event time, on the context's stream, of the kernels that order the
+                                    whole text: the prefix sort's rounds, or the top-level tile merge (a text
+                                    of at most 16 KiB: the host's time of its one kernel) */
+    int64_t merge_kernel_elements; /* elements that those ordered (the whole text) */
 } sadcs_stats;
 
-/* Construction parameters; zero fields take the defaults (of the cover, for G and tile threads). */
+/* Construction parameters; zero fields take the defaults (of the cover, for G and tile threads). A
+ * context with any of the three merge parameters set builds by the tile merge alone. Without them it
+ * also builds by one workgroup a text (all texts at most 16 KiB) and by the prefix sort (most others),
+ * which are faster; both order ties by cover 32 whatever the cover, and a context of one text of up
+ * to 48 MiB takes 22 bytes more per input byte, where they are free, to sort it in one round. */
 typedef struct sadcs_params {
     int32_t cover;               /* 32 (default) or 128 */
     uint32_t splitter_spacing;   /* G: every G-th element of a list is a splitter; 16 (cover 32), 8 (cover 128) */
@@ -149,7 +155,9 @@ int sadcs_hip_batch_build_device(sadcs_ctx* context, const void* d_texts, const 
  * threads 512 or 256, splitter spacing G in {8, 12, 16, 24, 32} (cover 128: {4, 6, 8, 12}) and tile splitters K at 1, 3/4 and
  * 1/2 of the most that keep the tiles a CU runs at once in its LDS - and writes the fastest (by device time, best of two builds) to *best; the
  * cover comes from base (null: 32). count 1: d_texts is one text of lengths[0] bytes followed by
- * 64 zero bytes; count > 1: a batch in the sadcs_hip_batch_layout layout. best_seconds may be null. */
+ * 64 zero bytes; count > 1: a batch in the sadcs_hip_batch_layout layout. best_seconds may be null.
+ * The configuration is the tile merge's, and a context given it takes no other path: for very
+ * repetitive texts. Most texts build faster without one. */
 int sadcs_hip_tune(const void* d_texts, const int64_t* lengths, int32_t count, const sadcs_params* base,
                    sadcs_params* best, double* best_seconds);
 

@@ -27,8 +27,9 @@
 namespace sadcs {
 
 // The largest text whose arrays fit the LDS of a CU beside the counters: 16384 bytes take 127 KB of
-// 160. At that size it is still the faster path alone, whatever the text: one long run 0.61 against
-// the phases' 1.27 ms, periodic 0.60 against 1.29, DNA-like 0.57 against 0.73, Markov 0.68 against 0.75.
+// 160. Alone at that size, against the prefix sort: protein-like 0.14 to 0.19 ms, DNA-like 0.47 to
+// 0.52, periodic 0.44 to 1.19, but Markov 0.53 to 0.30 (8192 bytes: 0.30 to 0.27); what a text is like
+// is not known here, and a batch of such texts has a workgroup for each.
 constexpr uint32_t kSmallMax = 16384;
 constexpr int kSmallBins = 256;
 
