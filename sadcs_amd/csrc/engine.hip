@@ -98,12 +98,6 @@ __global__ void fillWordsKernel(uint32_t* __restrict__ out, uint64_t count, uint
     }
 }
 
-__global__ void fillBytesKernel(uint8_t* __restrict__ out, uint64_t count, uint8_t value) {
-    for (uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < count; i += uint64_t(gridDim.x) * blockDim.x) {
-        out[i] = value;
-    }
-}
-
 // The bytes that occur in the texts, as a 256-bit mask (bit b mod 32 of word b / 32): the dense
 // codes need only which bytes occur, not how often. Each thread reads 16-byte chunks (the text
 // buffer is 16-byte aligned and padded); gap bytes between the texts of a batch are masked off (a

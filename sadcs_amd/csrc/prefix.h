@@ -21,9 +21,9 @@
  *     tile merge as class lists of their own.
  * Texts whose suffixes tie in large groups throughout keep the tile merge alone.
  *
- * Measured against the tile merge (SA + BWT on the device): 1 GiB of Markov text 100.1 to 66.0 ms,
- * 256 MiB of DNA-like text 31.8 to 22.1 ms (cover 128: 87.4 to 22.1), 16 MiB of uniform ACGT at
- * cover 128 4.07 to 1.26 ms, 1024 texts of 1 KiB to 4 MiB in one batch 62.3 to 45.2 ms.
+ * Measured against the tile merge (SA + BWT on the device): 1 GiB of Markov text 100.1 to 58.7 ms,
+ * 256 MiB of DNA-like text 31.8 to 18.6 ms (cover 128: 87.2 to 18.6), 16 MiB of uniform ACGT at
+ * cover 128 4.06 to 0.95 ms, 1024 texts of 1 KiB to 4 MiB in one batch 62.5 to 40.1 ms.
  */
 #pragma once
 

@@ -710,22 +710,21 @@ inline void radixPassDigits(hipStream_t stream, SortBuffers<K>& b, Source source
 // 1024 against 10; 53 us for 4096), a launch of the merge on its few probes of memory (4.7 us).
 
 constexpr int kChunkLane = 4;             // items a lane sorts in registers
-constexpr uint32_t kChunkWave = kWave * kChunkLane;
 constexpr int kChunkThreads = 256;
 constexpr uint32_t kChunk = kChunkThreads * kChunkLane;  // items a workgroup sorts
 constexpr uint32_t kRunTile = 1024;     // outputs of a workgroup of mergeRunsKernel
 constexpr int kRunThreads = 256;
 constexpr int kRunItems = kRunTile / kRunThreads;
 
-// One phase of the bitonic sort of a wave's kChunkWave items, item lane * kChunkLane + r in key[r],
-// index[r]: sorted runs of kRun / 2, alternately ascending and descending, into runs of kRun.
-template <int kRun, int kStride, class K>
-__device__ __forceinline__ void chunkStages(K (&key)[kChunkLane], uint32_t (&index)[kChunkLane], uint32_t lane) {
-    if constexpr (kStride >= kChunkLane) {
-        constexpr int kLanes = kStride / kChunkLane;
-        const bool keepSmaller = ((lane & kLanes) == 0) == ((lane & (kRun / kChunkLane)) == 0);
+// One phase of the bitonic sort of a wave's items, item lane * kLane + r in key[r], index[r]: sorted
+// runs of kRun / 2, alternately ascending and descending, into runs of kRun.
+template <int kRun, int kStride, class K, int kLane>
+__device__ __forceinline__ void itemStages(K (&key)[kLane], uint32_t (&index)[kLane], uint32_t lane) {
+    if constexpr (kStride >= kLane) {
+        constexpr int kLanes = kStride / kLane;
+        const bool keepSmaller = ((lane & kLanes) == 0) == ((lane & (kRun / kLane)) == 0);
 #pragma unroll
-        for (int r = 0; r < kChunkLane; r++) {
+        for (int r = 0; r < kLane; r++) {
             const K k = static_cast<K>(laneXor64<kLanes>(key[r]));
             const uint32_t i = laneXor<kLanes>(index[r]);
             const bool keep = ((key[r] < k) | ((key[r] == k) & (index[r] < i))) == keepSmaller;
@@ -734,9 +733,9 @@ __device__ __forceinline__ void chunkStages(K (&key)[kChunkLane], uint32_t (&ind
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < kChunkLane; r++) {
+        for (int r = 0; r < kLane; r++) {
             if ((r & kStride) == 0) {
-                const bool ascending = kRun >= kChunkLane ? (lane & (kRun / kChunkLane)) == 0 : (r & kRun) == 0;
+                const bool ascending = kRun >= kLane ? (lane & (kRun / kLane)) == 0 : (r & kRun) == 0;
                 const K ka = key[r], kb = key[r + kStride];
                 const uint32_t ia = index[r], ib = index[r + kStride];
                 const bool keep = ((ka < kb) | ((ka == kb) & (ia < ib))) == ascending;
@@ -748,26 +747,65 @@ __device__ __forceinline__ void chunkStages(K (&key)[kChunkLane], uint32_t (&ind
         }
     }
     if constexpr (kStride > 1) {
-        chunkStages<kRun, kStride / 2>(key, index, lane);
+        itemStages<kRun, kStride / 2>(key, index, lane);
     }
 }
 
-template <int kRun, class K>
-__device__ __forceinline__ void sortChunkWave(K (&key)[kChunkLane], uint32_t (&index)[kChunkLane], uint32_t lane) {
+template <int kRun, class K, int kLane>
+__device__ __forceinline__ void sortWaveItems(K (&key)[kLane], uint32_t (&index)[kLane], uint32_t lane) {
     if constexpr (kRun > 2) {
-        sortChunkWave<kRun / 2>(key, index, lane);
+        sortWaveItems<kRun / 2>(key, index, lane);
     }
-    chunkStages<kRun, kRun / 2>(key, index, lane);
+    itemStages<kRun, kRun / 2>(key, index, lane);
 }
 
-// Chunk blockIdx.x stably by the bits from beginBit on: a wave sorts 256 items in registers, by
-// (key, index), and the waves' runs merge in LDS.
+// Item threadIdx.x * kLane + r of a workgroup in key[r], index[r], the first `width` of them (a power of
+// two, at least a wave's) sorted by (key, index): a wave's in registers, the waves' runs merged through
+// LDS (`width` of each array). An item's index rises along the items.
+template <class K, int kLane>
+__device__ __forceinline__ void sortGroupItems(K (&key)[kLane], uint32_t (&index)[kLane], uint32_t width, K* shared, uint16_t* sharedIndex) {
+    const uint32_t o = threadIdx.x * kLane;
+    if (o < width) {
+        sortWaveItems<kWave * kLane>(key, index, laneId());
+    }
+    for (uint32_t run = kWave * kLane; run < width; run *= 2) {
+        __syncthreads();
+        if (o < width) {
+#pragma unroll
+            for (int r = 0; r < kLane; r++) {
+                shared[o + r] = key[r];
+                sharedIndex[o + r] = static_cast<uint16_t>(index[r]);
+            }
+        }
+        __syncthreads();
+        if (o < width) {
+            const uint32_t a = o / (2 * run) * (2 * run), b = a + run, d = o - a;
+            uint32_t lo = d > run ? d - run : 0, hi = min(d, run);
+            while (lo < hi) {
+                const uint32_t m = (lo + hi) / 2;
+                const bool take = shared[a + m] <= shared[b + d - 1 - m];
+                lo = take ? m + 1 : lo;
+                hi = take ? hi : m;
+            }
+            uint32_t x = lo, y = d - lo;
+#pragma unroll
+            for (int r = 0; r < kLane; r++) {
+                const bool take = x < run && (y >= run || shared[a + x] <= shared[b + y]);
+                const uint32_t from = take ? a + x++ : b + y++;
+                key[r] = shared[from];
+                index[r] = sharedIndex[from];
+            }
+        }
+    }
+}
+
+// Chunk blockIdx.x stably by the bits from beginBit on.
 template <class K>
 __global__ __launch_bounds__(kChunkThreads) void sortChunksKernel(const K* __restrict__ keys, const uint32_t* __restrict__ values, uint32_t count, int beginBit, K* __restrict__ keysOut, uint32_t* __restrict__ valuesOut) {
     __shared__ K shared[kChunk];
     __shared__ uint16_t sharedIndex[kChunk];
     const uint32_t first = blockIdx.x * kChunk, size = min(kChunk, count - first);
-    const uint32_t o = threadIdx.x * kChunkLane, lane = laneId();
+    const uint32_t o = threadIdx.x * kChunkLane;
     K key[kChunkLane];
     uint32_t index[kChunkLane];
 #pragma unroll
@@ -775,32 +813,7 @@ __global__ __launch_bounds__(kChunkThreads) void sortChunksKernel(const K* __res
         index[r] = o + r;
         key[r] = o + r < size ? keys[first + o + r] >> beginBit : ~K(0);  // past the end: the last of the largest
     }
-    sortChunkWave<kChunkWave>(key, index, lane);
-    for (uint32_t run = kChunkWave; run < kChunk; run *= 2) {
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kChunkLane; r++) {
-            shared[o + r] = key[r];
-            sharedIndex[o + r] = static_cast<uint16_t>(index[r]);
-        }
-        __syncthreads();
-        const uint32_t a = o / (2 * run) * (2 * run), b = a + run, d = o - a;
-        uint32_t lo = d > run ? d - run : 0, hi = min(d, run);
-        while (lo < hi) {
-            const uint32_t m = (lo + hi) / 2;
-            const bool take = shared[a + m] <= shared[b + d - 1 - m];
-            lo = take ? m + 1 : lo;
-            hi = take ? hi : m;
-        }
-        uint32_t x = lo, y = d - lo;
-#pragma unroll
-        for (int r = 0; r < kChunkLane; r++) {
-            const bool take = x < run && (y >= run || shared[a + x] <= shared[b + y]);
-            const uint32_t from = take ? a + x++ : b + y++;
-            key[r] = shared[from];
-            index[r] = sharedIndex[from];
-        }
-    }
+    sortGroupItems(key, index, kChunk, shared, sharedIndex);
 #pragma unroll
     for (int r = 0; r < kChunkLane; r++) {
         if (o + r < size) {

@@ -533,9 +533,12 @@ __global__ __launch_bounds__(256) void scatterResolvedRanksKernel(const uint32_t
 // the list, the group ids, the keys and the scans live in LDS, the workgroup loops until the list
 // is empty, and the host waits once. A pass is the same as above - the keys of makePassKeysKernel,
 // a sort by key, the mark scan of MarkConsumer - so ids, ranks and the sorted sample come out the
-// same. The sort is a bitonic network on (key, list index); ties among equal keys only reorder
-// members of one unresolved group, whose id they share.
-constexpr uint32_t kTailMax = 4096;  // list entries the workgroup takes
+// same. The sort is by (key, list index), each wave's entries in registers and the waves' runs merged
+// in LDS: as one bitonic network in LDS its 66 barriers took most of a pass (DNA-like text of 71,019
+// bytes 0.74 ms instead of 0.68). Lists of 4096 entries are slower here than by launches (Markov text
+// of 500,019 bytes 0.64 against 0.58 ms), those of 2048 faster (DNA-like, 871,019 bytes, to 1024 here:
+// 0.84 against 0.76).
+constexpr uint32_t kTailMax = 2048;  // list entries the workgroup takes
 constexpr int kTailThreads = 1024;
 constexpr int kTailItems = kTailMax / kTailThreads;  // consecutive sorted entries per thread in the scan
 
@@ -611,11 +614,17 @@ __global__ __launch_bounds__(kTailThreads) void rankTailKernel(TailParams tp, Te
         }
 
         // Keys (makePassKeysKernel after the first pass); entries past u sort last.
-        uint32_t width = 1;
+        uint32_t width = kWave * kTailItems;
         while (width < u) {
             width <<= 1;
         }
-        for (uint32_t i = tid; i < width; i += kTailThreads) {
+        uint64_t itemKey[kTailItems];
+        uint32_t itemIndex[kTailItems];
+#pragma unroll
+        for (int j = 0; j < kTailItems; j++) {
+            const uint32_t i = tid * kTailItems + j;
+            itemKey[j] = ~uint64_t(0);
+            itemIndex[j] = i;
             if (i < u) {
                 const uint32_t t = listT[cur][i];
                 const uint32_t p = unpackIndex<V>(t);
@@ -637,35 +646,20 @@ __global__ __launch_bounds__(kTailThreads) void rankTailKernel(TailParams tp, Te
                         subkey = (subkey << tp.charBits) | ch;
                     }
                 }
-                key[i] = (subkeyBits < 64 ? (uint64_t(listOrdinal[cur][i]) << subkeyBits) : 0) | subkey;
-                index[i] = static_cast<uint16_t>(i);
-            } else {
-                key[i] = ~uint64_t(0);
-                index[i] = 0xFFFF;
+                itemKey[j] = (subkeyBits < 64 ? (uint64_t(listOrdinal[cur][i]) << subkeyBits) : 0) | subkey;
+            }
+        }
+        sortGroupItems(itemKey, itemIndex, width, key, index);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kTailItems; j++) {
+            const uint32_t i = tid * kTailItems + j;
+            if (i < width) {
+                key[i] = itemKey[j];
+                index[i] = static_cast<uint16_t>(itemIndex[j]);
             }
         }
         __syncthreads();
-
-        // Bitonic sort of (key, index), ascending.
-        for (uint32_t k = 2; k <= width; k <<= 1) {
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                for (uint32_t i = tid; i < width; i += kTailThreads) {
-                    const uint32_t l = i ^ j;
-                    if (l > i) {
-                        const uint64_t a = key[i], b = key[l];
-                        const uint16_t ia = index[i], ib = index[l];
-                        const bool greater = a > b || (a == b && ia > ib);
-                        if (greater == ((i & k) == 0)) {
-                            key[i] = b;
-                            key[l] = a;
-                            index[i] = ib;
-                            index[l] = ia;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
 
         // The mark scan (MarkProducer/MarkConsumer) over sorted entries tid * kTailItems + 0..3.
         const int shift = subkeyBits < 64 ? subkeyBits : 0;
