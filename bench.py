@@ -18,7 +18,7 @@ Printed as one JSON line, with:
   e2e_hbm_fraction: the whole step's algorithmic bytes (127.94 bytes per input byte for fused
     SA + BWT) over the step time, against 8 TB/s;
   host_call: the same 1 GiB text through the host-memory API (pageable text in, SA and BWT out,
-    PCIe included; the download overlaps the end of the merge), best of 3 calls, outputs compared
+    PCIe included), best of 3 calls, outputs compared
     with the device-resident build's - a secondary figure, never value;
   cpu_baseline: the reference's CPU construction (oracle/_ref, OpenMP on all host threads, cover
     128) on the same whole text, SA and BWT built separately as the reference CLI does, best of 3
@@ -350,7 +350,7 @@ def host_call_measurement(ctx, text, d_sa, d_bwt, primary, runs):
     return {"value": round(n / wall / 1e6, 1), "unit": "MB/s", "ms": round(wall * 1e3, 1),
             "upload_ms": round(upload * 1e3, 1), "device_ms": round(device * 1e3, 1),
             "download_after_merge_ms": round(download * 1e3, 1), "runs": runs,
-            "io": "pageable host memory in and out over PCIe; the download overlaps the top-level merge",
+            "io": "pageable host memory in and out over PCIe",
             "outputs_equal_device_build": same}
 
 
