@@ -21,6 +21,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <thread>
 #include <vector>
 
@@ -3136,12 +3137,22 @@ int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sad
     const size_t count = layout.segments.size();
     const size_t total = static_cast<size_t>(layout.totalLength);
 
+    // The longest texts' workgroups start first: a CU takes one at a time, and a long one that starts
+    // last is waited for alone (512 documents of up to 16 KiB: the kernel 0.80 -> 0.63 ms).
+    std::vector<uint32_t> order(count);
+    std::iota(order.begin(), order.end(), 0u);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+        return layout.segments[x].end - layout.segments[x].start > layout.segments[y].end - layout.segments[y].start;
+    });
+
     // Chunk 1 holds the segment table, the first rows and the rounds; then small outputs.
     SADCS_HIP(hipStreamSynchronize(ctx.stream));
     Segment* segments = reinterpret_cast<Segment*>(ctx.staging[1]);
     uint32_t* firstRows = reinterpret_cast<uint32_t*>(segments + count);
     uint32_t* rounds = firstRows + count;
-    std::copy(layout.segments.begin(), layout.segments.end(), segments);
+    for (size_t k = 0; k < count; k++) {
+        segments[k] = layout.segments[order[k]];
+    }
     *rounds = 0;
     const size_t tableBytes = (count * (sizeof(Segment) + sizeof(uint32_t)) + sizeof(uint32_t) + 255) / 256 * 256;
 
@@ -3206,8 +3217,8 @@ int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sad
     const double deviceSeconds = secondsSince(deviceStart);
 
     if (wantBWT && rq.hostPrimaries) {
-        for (size_t i = 0; i < count; i++) {
-            rq.hostPrimaries[i] = static_cast<int32_t>(firstRows[i]) + 1;
+        for (size_t k = 0; k < count; k++) {
+            rq.hostPrimaries[order[k]] = static_cast<int32_t>(firstRows[k]) + 1;
         }
     }
     PhaseTimes times;
