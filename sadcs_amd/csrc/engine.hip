@@ -1748,6 +1748,7 @@ class Pipeline {
             tileOut.index = order;
             const int status = mergeLevel<kOutIndex>(lists, tileOut, errors);
             if (status == SADCS_NOT_ENOUGH_MEMORY) {
+                tLastError[0] = '\0';  // the tile merge takes the text: no failure of the call
                 releaseTaken();
                 return SADCS_OK;
             }
@@ -2407,9 +2408,21 @@ size_t planBytes(const sadcs_ctx& base, const Layout& layout, Mode mode, bool ow
     if (status != SADCS_OK) {
         return SIZE_MAX;
     }
-    // A text below 1 MiB is bound by launches, not by memory: room for the prefix sort in one round.
-    const size_t roomy = mode != Mode::RankOnly && layout.span < (uint32_t(1) << 20) ? size_t(1) << 19 : 0;
-    return std::max(ctx.arena.highWater(), roomy ? roomy + (ownOutputs ? 32 : 26) * static_cast<size_t>(layout.span) : 0);
+    return ctx.arena.highWater();
+}
+
+// Beyond its plan a context for up to kRoomyText bytes of text takes kRoomyBytes more a byte, if that is
+// a small part of the free memory: the prefix sort then holds all records at once instead of reading
+// the text once a round (8 MiB: one round instead of five). It is never part of a plan, which decides
+// what a context, a call or a server's budget has to hold. A context that serves one call, and a batch
+// of a server, take it below kRoomyOnce only: rounds over texts that short are bound by their launches.
+constexpr uint64_t kRoomyText = uint64_t(48) << 20;
+constexpr uint64_t kRoomyOnce = uint64_t(1) << 20;
+constexpr uint64_t kRoomyBytes = 22;
+
+size_t roomyBytes(const Params& params, uint64_t text, uint64_t most = kRoomyText) {
+    // Merge parameters select the tile merge; one workgroup's texts need no such memory.
+    return params.tiles || text <= kSmallMax || text > most ? 0 : static_cast<size_t>((uint64_t(1) << 19) + text * kRoomyBytes);
 }
 
 size_t planFor(const sadcs_ctx& base, const Layout& layout, Mode mode, bool ownText, bool ownOutputs) {
@@ -2778,16 +2791,6 @@ int downloadSlices(sadcs_ctx& ctx, const OutputSlices& o) {
     }
     SADCS_HIP(hipStreamSynchronize(ctx.copyStream));
     return SADCS_OK;
-}
-
-// Beyond its plan a context for up to this many bytes of text takes kRoomyBytes more a byte, if that is
-// a small part of the free memory: the prefix sort then holds all records at once instead of reading
-// the text once a round (8 MiB: one round instead of five).
-constexpr int64_t kRoomyText = int64_t(48) << 20;
-constexpr int64_t kRoomyBytes = 22;
-
-size_t roomyBytes(int64_t text) {
-    return text <= kRoomyText ? static_cast<size_t>(text * kRoomyBytes) : 0;
 }
 
 int createContext(size_t arenaBytes, const Params& params, int32_t capacity, sadcs_ctx*& out, size_t optional = 0) {
@@ -3321,7 +3324,7 @@ int buildOn(sadcs_ctx* context, const Params& params, const Layout& layout, cons
         return SADCS_FAILED;
     }
     sadcs_ctx* ctx = nullptr;
-    SADCS_TRY(createContext(need, params, 0, ctx));
+    SADCS_TRY(createContext(need, params, 0, ctx, rq.mode == Mode::RankOnly ? 0 : roomyBytes(params, layout.span, kRoomyOnce)));
     const double setup = secondsSince(start);
     const int status = build(*ctx, layout, rq, stats);
     if (stats) {
@@ -3518,7 +3521,7 @@ int sadcs_hip_ctx_create_batch(const int64_t* lengths, int32_t count, const sadc
         setError("planning the device memory failed");
         return SADCS_FAILED;
     }
-    return createContext(plan, p, static_cast<int32_t>(longest), *context, p.tiles ? 0 : roomyBytes(total));
+    return createContext(plan, p, static_cast<int32_t>(longest), *context, roomyBytes(p, total));
 }
 
 int sadcs_hip_ctx_create(int32_t capacity, const sadcs_params* params, sadcs_ctx** context) {
@@ -3542,7 +3545,7 @@ int sadcs_hip_ctx_create(int32_t capacity, const sadcs_params* params, sadcs_ctx
         setError("planning the device memory failed");
         return SADCS_FAILED;
     }
-    return createContext(plan, p, std::max(capacity, 0), *context, p.tiles ? 0 : roomyBytes(std::max(capacity, 0)));
+    return createContext(plan, p, std::max(capacity, 0), *context, roomyBytes(p, std::max(capacity, 0)));
 }
 
 void sadcs_hip_ctx_destroy(sadcs_ctx* context) {
@@ -4302,7 +4305,7 @@ class Server {
         return m_wantSA && m_wantBWT ? Mode::Both : m_wantSA ? Mode::SA : Mode::BWT;
     }
 
-    size_t planOf(const std::vector<std::shared_ptr<ServerRequest>>& batch) {
+    size_t planOf(const std::vector<std::shared_ptr<ServerRequest>>& batch, size_t& optional) {
         std::vector<int64_t> lengths;
         for (auto& r : batch) {
             lengths.push_back(static_cast<int64_t>(r->text.size));
@@ -4310,6 +4313,7 @@ class Server {
         const Layout layout = layoutFor(m_params, lengths.data(), static_cast<int32_t>(lengths.size()), batch.size() > 1);
         sadcs_ctx planner;
         planner.params = m_params;
+        optional = roomyBytes(m_params, layout.span, kRoomyOnce);
         return planFor(planner, layout, mode(), true, true);
     }
 
@@ -4355,7 +4359,8 @@ class Server {
             total += r->text.size + kSegmentAlign;
         }
         while (!batch.empty()) {
-            const size_t plan = planOf(batch);
+            size_t optional = 0;
+            const size_t plan = planOf(batch, optional);
             if (plan == SIZE_MAX) {
                 batch.clear();
                 break;
@@ -4366,6 +4371,12 @@ class Server {
                 break;
             }
             uint8_t* p = nullptr;
+            // The optional memory from a pool of which it is a small part, so that it keeps no one waiting.
+            if (optional > 0 && plan + optional <= m_budget / 8 && m_pool.tryAllocate(p, plan + optional)) {
+                chunk = p;
+                bytes = plan + optional;
+                return batch;
+            }
             if (plan <= m_budget && m_pool.allocate(p, plan) == SADCS_OK) {
                 chunk = p;
                 bytes = plan;

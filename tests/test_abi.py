@@ -78,3 +78,15 @@ def test_gather_calibration_refuses_bad_arguments():
     assert lib.sadcs_hip_gather_lines(ctypes.c_void_p(16), 0, 10, 1) == sadcs_amd.GpuStatus.Failed
     assert lib.sadcs_hip_gather_lines(ctypes.c_void_p(16), 1 << 32, 10, 1) == sadcs_amd.GpuStatus.Failed
     assert "gather_lines" in sadcs_amd.gpu_last_error()
+
+
+def test_plan_grows_with_the_text():
+    """What a context for a longer text holds, and a budget that admits one, is enough for a shorter one:
+    memory that only makes a short text faster is not in its plan."""
+    sizes = [1 << 18, 500_000, 900_000, (1 << 20) - 1, 1 << 20, 2_000_000]
+    for plan in (sadcs_amd.gpu_required_bytes, lambda n: sadcs_amd.lib.sadcs_hip_device_required_bytes(n, 1, 1)):
+        plans = [plan(n) for n in sizes]
+        assert plans == sorted(plans), plans
+    lengths = [np.array([n // 3] * 3, dtype=np.int64) for n in sizes]
+    plans = [sadcs_amd.lib.sadcs_hip_batch_required_bytes(l.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), 3) for l in lengths]
+    assert plans == sorted(plans), plans

@@ -152,3 +152,19 @@ def test_cover_128_by_cover_32(gpu, n):
         assert gpu.gpu_check_device(d_text.ptr, n, d_sa.ptr, d_bwt.ptr, primary) == (0, -1)
         sa, bwt, got = check_device(gpu, text, cover=128)
         assert np.array_equal(sa, d_sa.to_host(np.int32)) and bwt == d_bwt.to_host(np.uint8).tobytes() and got == primary
+
+
+@pytest.mark.parametrize("n", [700_001, (1 << 20) - 1])
+def test_short_text_in_what_a_longer_one_needs(gpu, n):
+    # A context with merge parameters holds its plan and no more; a server's budget of twelve bytes a byte
+    # leaves nothing beyond the plan. Both take the text, as does a context of its own.
+    text = text_of("protein", n)
+    want, bwt, primary = check_device(gpu, text)
+    with gpu.GpuContext(1 << 20, tile_splitters=8) as ctx:
+        sa, b, p = gpu.gpu_build(text, True, True, context=ctx)
+    assert np.array_equal(sa, want) and (b, p) == (bwt, primary)
+    with gpu.Server(memory_budget=12 << 20, workers=1) as server:
+        sa, b, p, *_ = server.wait(server.submit(text))
+    assert np.array_equal(sa, want) and (b, p) == (bwt, primary)
+    sa, b, p = gpu.gpu_build(text, True, True)
+    assert np.array_equal(sa, want) and (b, p) == (bwt, primary)
