@@ -907,8 +907,8 @@ inline void mergeSort(hipStream_t stream, SortBuffers<K>& b, uint32_t count, int
     }
 }
 
-// Up to here the merges win: half a million 64-bit keys of periodic text 2.08 against 2.31 ms for the
-// whole build, 12,000 of them 0.70 against 1.10 ms; at a million the two are even.
+// Up to here the merges win: half a million 64-bit keys of periodic text 2.04 against 2.31 ms for the
+// whole build, 12,000 of them 0.76 against 1.10 ms; at a million the two are even.
 constexpr uint32_t kMergeSortMax = 1 << 19;
 
 // Stable sort of b.keys[current], b.values[current] (count items) by bits [beginBit, endBit); the bits

@@ -16,7 +16,7 @@
  *
  * What bounds it: the barriers and LDS round trips of one workgroup's digit passes, and for a host
  * call the call's own launch and wait. Measured (host calls, SA + BWT, phases against this): 4099
- * bytes of protein 530 to 74 us; 512 documents of 200 B to 16 KiB in one batch 11.5 to 2.6 ms.
+ * bytes of protein 507 to 74 us; 512 documents of 200 B to 16 KiB in one batch 10.9 to 2.5 ms.
  */
 #pragma once
 
