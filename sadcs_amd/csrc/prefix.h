@@ -31,6 +31,7 @@
 #include <cstdint>
 #include "dev_common.h"
 #include "merge.h"
+#include "prefix_plan.h"
 #include "prim.h"
 #include "rank.h"
 
@@ -360,7 +361,7 @@ __device__ __forceinline__ uint32_t blockKeys(const PrefixText& pt, const Texts&
     uint64_t high = static_cast<uint64_t>(window >> 64), low = static_cast<uint64_t>(window);
     if constexpr (Texts::kBatch) {
         // Codes of the next text are not this one's.
-        const uint32_t held = min(remaining * bits, 128u);
+        const uint32_t held = heldBits(remaining, bits);
         high &= held >= 64 ? ~uint64_t(0) : ~(~uint64_t(0) >> held);
         low &= held >= 128 ? ~uint64_t(0) : held <= 64 ? 0 : ~(~uint64_t(0) >> (held - 64));
     }
