@@ -3129,7 +3129,7 @@ int launchSmallTexts(hipStream_t stream, uint32_t texts, const uint8_t* text, co
 // ask for the tile merge), and room for the tables in the pinned chunks.
 bool isSmall(const sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq) {
     return layout.maxLength <= kSmallMax && rq.mode != Mode::RankOnly && !ctx.params.tiles && ctx.staging[0] && ctx.staging[1] &&
-           layout.segments.size() * (sizeof(Segment) + sizeof(uint32_t)) + 4096 <= kStagingChunk / 2;
+           layout.segments.size() * (sizeof(Segment) + 2 * sizeof(uint32_t)) + 4096 <= kStagingChunk / 2;
 }
 
 int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sadcs_stats* stats) {
@@ -3156,8 +3156,7 @@ int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sad
     for (size_t k = 0; k < count; k++) {
         segments[k] = layout.segments[order[k]];
     }
-    *rounds = 0;
-    const size_t tableBytes = (count * (sizeof(Segment) + sizeof(uint32_t)) + sizeof(uint32_t) + 255) / 256 * 256;
+    const size_t tableBytes = (count * (sizeof(Segment) + 2 * sizeof(uint32_t)) + 255) / 256 * 256;
 
     const auto uploadStart = std::chrono::steady_clock::now();
     const uint8_t* text = rq.deviceText;
@@ -3229,7 +3228,7 @@ int buildSmall(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, sad
     times.mergeKernel = deviceSeconds;
     times.mergeElements = layout.totalLength;
     times.characterPasses = 1;
-    times.doublingRounds = static_cast<int>(*rounds);
+    times.doublingRounds = static_cast<int>(*std::max_element(rounds, rounds + count));
     times.rankingBytes = times.classBytes = times.mergeBytes = arena.highWater();
     const auto downloadStart = std::chrono::steady_clock::now();
     if (!deviceCall) {
