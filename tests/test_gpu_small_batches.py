@@ -42,7 +42,8 @@ def best_ms(gpu, lengths, **params):
     return best * 1e3, outputs
 
 
-@pytest.mark.parametrize("lengths", [[1024] * 16_000], ids=["16000 of 1 KiB"])
+@pytest.mark.parametrize("lengths", [[1024] * 16_000, [100] * 100_000 + [16_384], [16_384, 2049] + [2048, 1] * 1024, [300] * 2047 + [5000]],
+                         ids=["16000 of 1 KiB", "100000 of 100 B and one of 16 KiB", "2048 short, two long", "2047 short, one long"])
 def test_many_short_texts_against_the_tile_merge(gpu, lengths):
     small, outputs = best_ms(gpu, lengths)
     tiles, want = best_ms(gpu, lengths, splitter_spacing=16)  # its default parameters
