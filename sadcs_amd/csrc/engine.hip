@@ -505,7 +505,7 @@ struct sadcs_ctx {
 namespace sadcs {
 
 constexpr size_t kStagingChunk = size_t(32) << 20;
-// Pinned readback words: [0, 2050) the prefix sort's bucket rows, [0, 16) counters, [16, 1016) the first rows of a batch (after the build), [kSliceRowWords, +kSlices + 1)
+// Pinned readback words: [0, 2052) the prefix sort's bucket rows, [0, 16) counters, [16, 1016) the first rows of a batch (after the build), [kSliceRowWords, +kSlices + 1)
 // the row bounds of the top-level merge's slices.
 constexpr size_t kHostWords = 4096;
 constexpr size_t kSliceRowWords = 1024;
@@ -552,6 +552,11 @@ constexpr uint64_t kGroupRankMeanMax = 8;
 
 // Lists up to this long are scanned while the host does not know yet whether all of it is sorted.
 constexpr uint32_t kGuessMax = 1 << 20;
+
+// Of a row as a class list entry of the prefix sort's large tie groups, with the merge's own levels; and
+// what these take of any list.
+constexpr uint64_t kLargeTieBytes = 38;
+constexpr uint64_t kMergeRoom = 1 << 16;
 
 // Lists up to this long are doubled with every id that fits the key.
 constexpr uint32_t kWideKeysMax = 1 << 18;
@@ -1119,7 +1124,7 @@ class Pipeline {
     // ---- the prefix-sort path (prefix.h) ---------------------------------------------------------
 
     // Device words read back by the host in one copy.
-    enum : uint32_t { kReadEqual = 0, kReadBigLeaves = 1, kReadBigRecords = 2, kReadLarge = 3, kReadWords = 8 };
+    enum : uint32_t { kReadSeen = 0, kReadBigLeaves = kSeenWords, kReadBigRecords, kReadLarge, kReadWords = 8 };
 
     // The whole build by prefix sort. done = false, with nothing allocated left, where the tile merge
     // is the better path or the memory planned for this call does not hold this one.
@@ -1213,7 +1218,7 @@ class Pipeline {
 
         bool room = (m_job.sa || take(b.sa, m_job.span)) && (!m_job.wantBWT || m_job.bwt || take(b.bwt, m_job.span)) &&
                     take(b.ties, tieWords + 4) && take(b.words, kReadWords) && take(b.startKeys, m_segments) && take(b.bigList, kBigLeavesMax) &&
-                    take(b.splitters, leaves) && take(b.tableRows, kPrefixMaxBuckets + 2) && (m_job.firstRows || take(b.firstRows, m_segments));
+                    take(b.splitters, leaves) && take(b.tableRows, kPrefixMaxBuckets + 1 + kSeenWords) && (m_job.firstRows || take(b.firstRows, m_segments));
         const bool ownCodes = kBatch && m_segments > 1 && sigma < 256;
         if (ownCodes) {
             room = room && take(b.textMasks, static_cast<uint64_t>(m_segments) * 8) && take(b.textCodes, static_cast<uint64_t>(m_segments) * 256) &&
@@ -1355,9 +1360,32 @@ class Pipeline {
                 radixSort<uint64_t>(m_stream, sb, samples, 64 - kPrefixKeyBits, 64);
                 sample = sb.keys[sb.current];
             }
-            pickSplittersKernel<<<std::min<unsigned>(blocksFor(std::max(samples, leaves)), 1024), 256, 0, m_stream>>>(sample, samples, leaves, splitters, words + kReadEqual);
+            pickSplittersKernel<<<std::min<unsigned>(blocksFor(std::max(samples, leaves)), 1024), 256, 0, m_stream>>>(sample, samples, leaves, splitters, words + kReadSeen);
             SADCS_HIP(hipGetLastError());
             releaseTaken(0);
+        }
+
+        // Whether the sample has so many rows tie that the tile merge is the better path, or the only one.
+        auto leavesToMerge = [&](const uint32_t* seen) {
+            const double sampled = static_cast<double>(samples) * N / m_job.span;
+            if (seen[0] * static_cast<double>(kLeafTieShare) > sampled) {
+                return true;
+            }
+            const TieEstimate ties = estimateTies(sampled, seen[1], seen[2], static_cast<double>(samples) / m_job.span);
+            const bool large = ties.groupRows > 1.25 * kTieGroupMax;  // the estimate spreads that far
+            const uint64_t tied = static_cast<uint64_t>(ties.share * N), unresolved = static_cast<uint64_t>(ties.share * m_samples);
+            return (large && ties.share > (N >= kLongTies ? kLargeTieShare : kLargeTieShareShort)) ||
+                   !tiesFit(tied, large ? tied : 0, unresolved, budget - std::min<uint64_t>(budget, m_arena.live()));
+        };
+        // A long text is not read for its bucket counts first (256 MiB: 0.7 of the merge's 54 ms), a shorter
+        // one's host waits once (64 MiB: 0.03 of 3.2 ms).
+        const bool lookFirst = N >= (uint64_t(1) << 27);
+        if (lookFirst) {
+            SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, words + kReadSeen, kSeenWords * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+            SADCS_HIP(hipStreamSynchronize(m_stream));
+            if (leavesToMerge(m_ctx.hostWords)) {
+                return SADCS_OK;
+            }
         }
 
         // Bucket counts of the tiles, and from them the buckets' first rows.
@@ -1374,13 +1402,12 @@ class Pipeline {
         }
         countBucketsKernel<Texts><<<tiles, kPrefixThreads, 0, m_stream>>>(pt, m_texts, codes, splitters, buckets, bins, steps, tileBlocks, tiles, offsets);
         exclusiveSum(m_stream, offsets, offsets, static_cast<uint32_t>(offsetWords), offsetAggregates);
-        bucketRowsKernel<<<blocksFor(buckets + 2), 256, 0, m_stream>>>(offsets, tiles, buckets, static_cast<uint32_t>(N), words + kReadEqual, tableRows);
+        bucketRowsKernel<<<blocksFor(buckets + 1 + kSeenWords), 256, 0, m_stream>>>(offsets, tiles, buckets, static_cast<uint32_t>(N), words + kReadSeen, tableRows);
         SADCS_HIP(hipGetLastError());
-        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, tableRows, (buckets + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipMemcpyAsync(m_ctx.hostWords, tableRows, (buckets + 1 + kSeenWords) * sizeof(uint32_t), hipMemcpyDeviceToHost, m_stream));
         SADCS_HIP(hipStreamSynchronize(m_stream));
-        const std::vector<uint32_t> rows(m_ctx.hostWords, m_ctx.hostWords + buckets + 2);
-        // Sampled keys with 16 equal ones after them: their rows tie in groups of half a leaf or more.
-        if (static_cast<uint64_t>(rows[buckets + 1]) * kLargeTieShare > samples) {
+        const std::vector<uint32_t> rows(m_ctx.hostWords, m_ctx.hostWords + buckets + 1 + kSeenWords);
+        if (!lookFirst && samples > 0 && leavesToMerge(&rows[buckets + 1])) {
             releaseTaken(0);
             return SADCS_OK;
         }
@@ -1541,6 +1568,15 @@ class Pipeline {
         return SADCS_OK;
     }
 
+    // Whether `room` bytes hold what follows the sort: beside the ranks the lists of `unresolved` samples
+    // and their passes, then the tied rows, `large` of them as class lists.
+    bool tiesFit(uint64_t tied, uint64_t large, uint64_t unresolved, uint64_t room) const {
+        const uint64_t ranks = sizeof(uint32_t) * static_cast<uint64_t>(DifferenceCover<V>::pack(m_job.span));
+        const uint64_t lists = 8 * static_cast<uint64_t>(m_samples) + 14 * unresolved;
+        const uint64_t order = 5 * tied + kLargeTieBytes * large;
+        return ranks + std::max({lists, 30 * unresolved, order}) + kMergeRoom <= room;
+    }
+
     // Step 4: the ranks of the sample suffixes (m_ranks). tied: rows that tie with a neighbour.
     int prefixRank(const CodeTable& codes, int charBits, int chars, const RowOut& out, uint32_t tieWords, uint32_t& tied, uint64_t budget, bool& ranked) {
         static_assert(V == 32, "the sample's ranks order ties within 32 characters");
@@ -1572,17 +1608,19 @@ class Pipeline {
                 taken.pop_back();
             }
         };
+        const uint64_t roomBefore = budget - std::min<uint64_t>(budget, m_arena.live());
         const uint64_t rankWords = static_cast<uint64_t>(DifferenceCover<V>::pack(m_job.span)) + CoverSet<V>::kSize + 8;
         uint32_t *index = nullptr, *group = nullptr, *counts = nullptr;
         SampleVec* sampleAggregates = nullptr;
         GroupVec* groupAggregates = nullptr;
-        Sum1* tieAggregates = nullptr;
-        const uint64_t tieBytes = scanScratchBytes<Sum1, kSumItems>(tieWords);
+        using TieCounts = Vec<2, 0u>;
+        TieCounts* tieAggregates = nullptr;
+        const uint64_t tieBytes = scanScratchBytes<TieCounts, kSumItems>(tieWords);
         if (m_arena.live() + rankWords * sizeof(uint32_t) + Arena::kAlign > budget || !m_arena.tryAllocate(m_ranks, rankWords)) {
             return SADCS_OK;
         }
         bool room = take(index, M) && take(group, M) && take(counts, 8) && take(sampleAggregates, scanScratchBytes<SampleVec, kSampleItems>(N) / sizeof(SampleVec) + 1) &&
-                    take(groupAggregates, scanScratchBytes<GroupVec, kMarkItems>(M) / sizeof(GroupVec) + 1) && take(tieAggregates, tieBytes / sizeof(Sum1) + 1);
+                    take(groupAggregates, scanScratchBytes<GroupVec, kMarkItems>(M) / sizeof(GroupVec) + 1) && take(tieAggregates, tieBytes / sizeof(TieCounts) + 1);
         if (!room) {
             releaseTaken();
             return SADCS_OK;
@@ -1592,15 +1630,15 @@ class Pipeline {
         scanPipeline<SampleVec, kSampleItems>(m_stream, N, SampleProducer<V>{out.sa, out.ties}, SampleConsumer<V>{out.sa, index, group, M}, sampleAggregates);
         const GroupProducer groups{group, M};
         scanReduce<GroupVec, kMarkItems>(m_stream, M, groups, groupAggregates);
-        scanReduce<Sum1, kSumItems>(m_stream, tieWords, TieProducer{out.ties}, tieAggregates);
+        scanReduce<TieCounts, kSumItems>(m_stream, tieWords, TieCountProducer{out.ties}, tieAggregates);
         SADCS_HIP(hipGetLastError());
         // The totals: past the scanned aggregates, or the sums of a few tiles' own.
         GroupVec* groupHost = reinterpret_cast<GroupVec*>(m_ctx.hostWords);
-        Sum1* tieHost = reinterpret_cast<Sum1*>(m_ctx.hostWords + 1024);
+        TieCounts* tieHost = reinterpret_cast<TieCounts*>(m_ctx.hostWords + 1024);
         const uint32_t groupTiles = scanTiles<kMarkItems>(M), tieTiles = scanTiles<kSumItems>(tieWords);
         const bool groupFew = groupTiles <= kScanThreads, tieFew = tieTiles <= kScanThreads;
         SADCS_HIP(hipMemcpyAsync(groupHost, groupAggregates + (groupFew ? 0 : groupTiles), (groupFew ? groupTiles : 1) * sizeof(GroupVec), hipMemcpyDeviceToHost, m_stream));
-        SADCS_HIP(hipMemcpyAsync(tieHost, tieAggregates + (tieFew ? 0 : tieTiles), (tieFew ? tieTiles : 1) * sizeof(Sum1), hipMemcpyDeviceToHost, m_stream));
+        SADCS_HIP(hipMemcpyAsync(tieHost, tieAggregates + (tieFew ? 0 : tieTiles), (tieFew ? tieTiles : 1) * sizeof(TieCounts), hipMemcpyDeviceToHost, m_stream));
         SADCS_HIP(hipStreamSynchronize(m_stream));
         uint32_t unresolved = 0, unresolvedGroups = 0;
         for (uint32_t x = 0; x < (groupFew ? groupTiles : 1); x++) {
@@ -1608,8 +1646,15 @@ class Pipeline {
             unresolvedGroups += groupHost[x].v[2];
         }
         tied = 0;
+        uint32_t large = 0;
         for (uint32_t x = 0; x < (tieFew ? tieTiles : 1); x++) {
             tied += tieHost[x].v[0];
+            large += tieHost[x].v[1];
+        }
+        // Nothing is ranked for rows that would not be ordered.
+        if (!tiesFit(tied, large, unresolved, roomBefore)) {
+            releaseTaken();
+            return SADCS_OK;
         }
 
         RankPassState state;
@@ -1712,7 +1757,7 @@ class Pipeline {
                 room = room && take(keys[i], large) && take(values[i], large);
             }
             // The merge's own levels: splitters, rows and counts of about half a word per element.
-            if (!room || m_arena.live() + static_cast<uint64_t>(large) + (1u << 20) > budget) {
+            if (!room || m_arena.live() + static_cast<uint64_t>(large) + kMergeRoom > budget) {
                 releaseTaken();
                 return SADCS_OK;
             }

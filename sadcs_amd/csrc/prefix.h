@@ -57,8 +57,14 @@ constexpr uint32_t kOversample = 32;
 constexpr uint32_t kSmallLeaf = 512;
 constexpr uint32_t kCoarseLeaf = 1536;
 constexpr uint32_t kCoarseOversample = 16;
-constexpr uint32_t kTieGroupMax = 24;              // rows of a group compared in LDS
-constexpr uint64_t kLargeTieShare = 16;            // at most 1 / this of the sample in large groups
+constexpr uint64_t kLeafTieShare = 16;             // at most 1 / this of the sample in groups of half a leaf
+// The most of the rows, as the sample has it, in groups beyond kTieGroupMax, of long texts (from kLongTies
+// rows on) and of shorter ones, whose time is more in launches. Such a row costs 0.34 ns as a class list
+// entry; the tile merge of the whole text costs 0.04 ns a row more than the other steps here. Protein-like
+// text with near-copies of a piece, prefix sort and tile merge: 48 MiB, 0.1 of it 6.1 and 7.3 ms, 0.2 8.3
+// and 7.9, 0.5 15.0 and 9.6; 0.7 MB, 0.2 of it 0.86 and 0.95 ms, 0.4 1.11 and 1.10.
+constexpr double kLargeTieShare = 0.125, kLargeTieShareShort = 0.5;
+constexpr uint64_t kLongTies = uint64_t(1) << 23;
 
 // A suffix on its way to its row: its key (the character before it in the low byte) and position, 12
 // bytes together, so that a run of records is one run of memory: keys and positions apart wrote a
@@ -195,9 +201,9 @@ __global__ __launch_bounds__(256) void placeSampleKernel(const uint64_t* __restr
 }
 
 // splitters[x] (x in [0, leaves - 1)) = the sorted sample's key at (x + 1) / leaves of its valid
-// part; equal[0] counts sampled keys equal to the one kCoarseOversample places on: a group of that key
-// holds about a leaf of rows or more.
-__global__ __launch_bounds__(256) void pickSplittersKernel(const uint64_t* __restrict__ sorted, uint32_t count, uint32_t leaves, uint64_t* __restrict__ splitters, uint32_t* __restrict__ equal) {
+// part. seen counts sampled keys: [0] equal to the one kCoarseOversample places on (a group of that key holds
+// about half a leaf of rows or more), [1] equal to another, [2] to two others or more.
+__global__ __launch_bounds__(256) void pickSplittersKernel(const uint64_t* __restrict__ sorted, uint32_t count, uint32_t leaves, uint64_t* __restrict__ splitters, uint32_t* __restrict__ seen) {
     uint32_t lo = 0, hi = count;  // the valid keys come before the ~0 ones
     while (lo < hi) {
         const uint32_t mid = (lo + hi) / 2;
@@ -207,18 +213,38 @@ __global__ __launch_bounds__(256) void pickSplittersKernel(const uint64_t* __res
             hi = mid;
         }
     }
-    uint32_t ties = 0;
+    __shared__ uint32_t all[3];
+    if (threadIdx.x < 3) {
+        all[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    uint32_t counts[3] = {};
     for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < max(count, leaves); x += gridDim.x * blockDim.x) {
         if (x + 1 < leaves) {
             splitters[x] = lo > 0 ? sorted[static_cast<uint64_t>(lo) * (x + 1) / leaves] : ~uint64_t(0);
         }
-        ties += x + kCoarseOversample < lo && sorted[x] == sorted[x + kCoarseOversample] ? 1 : 0;
+        if (x < lo) {
+            const uint64_t own = sorted[x], far = sorted[min(x + kCoarseOversample, lo - 1)];
+            const uint64_t after = sorted[min(x + 1, lo - 1)], after2 = sorted[min(x + 2, lo - 1)];
+            const uint64_t before = sorted[max(x, 1u) - 1], before2 = sorted[max(x, 2u) - 2];
+            const bool a1 = x + 1 < lo && after == own, b1 = x > 0 && before == own;
+            counts[0] += x + kCoarseOversample < lo && far == own ? 1 : 0;
+            counts[1] += (a1 | b1) ? 1 : 0;
+            counts[2] += ((a1 & b1) | (x + 2 < lo && after2 == own) | (x > 1 && before2 == own)) ? 1 : 0;
+        }
     }
-    for (int offset = kWave / 2; offset > 0; offset /= 2) {
-        ties += __shfl_xor(ties, offset);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        for (int offset = kWave / 2; offset > 0; offset /= 2) {
+            counts[k] += __shfl_xor(counts[k], offset);
+        }
+        if (threadIdx.x % kWave == 0 && counts[k]) {
+            atomicAdd(&all[k], counts[k]);
+        }
     }
-    if (threadIdx.x % kWave == 0 && ties) {
-        atomicAdd(equal, ties);
+    __syncthreads();
+    if (threadIdx.x < 3 && all[threadIdx.x]) {
+        atomicAdd(&seen[threadIdx.x], all[threadIdx.x]);
     }
 }
 
@@ -453,16 +479,18 @@ __global__ __launch_bounds__(kPrefixThreads) void countBucketsKernel(PrefixText 
     }
 }
 
-// out[b] = the first row of bucket b (b = buckets: all rows), out[buckets + 1] = *equal: what the host
-// reads to plan the rounds.
-__global__ void bucketRowsKernel(const uint32_t* __restrict__ offsets, uint32_t tiles, uint32_t buckets, uint32_t allRows, const uint32_t* __restrict__ equal, uint32_t* __restrict__ out) {
+// out[b] = the first row of bucket b (b = buckets: all rows), and after them the sample's kSeenWords
+// counts: what the host reads to plan the rounds.
+constexpr uint32_t kSeenWords = 3;
+
+__global__ void bucketRowsKernel(const uint32_t* __restrict__ offsets, uint32_t tiles, uint32_t buckets, uint32_t allRows, const uint32_t* __restrict__ seen, uint32_t* __restrict__ out) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < buckets) {
         out[b] = offsets[static_cast<uint64_t>(b) * tiles];
     } else if (b == buckets) {
         out[b] = allRows;
-    } else if (b == buckets + 1) {
-        out[b] = *equal;
+    } else if (b <= buckets + kSeenWords) {
+        out[b] = seen[b - buckets - 1];
     }
 }
 
@@ -1279,6 +1307,18 @@ struct TieProducer {
     __device__ Vec<1, 0u> operator()(uint32_t w) const {
         Vec<1, 0u> r;
         r.v[0] = __builtin_popcount(tiedRows(ties[w], ties[w + 1]));
+        return r;
+    }
+};
+
+// Fields: rows that tie with a neighbour, rows of groups beyond kTieGroupMax.
+struct TieCountProducer {
+    const uint32_t* ties;
+    __device__ Vec<2, 0u> operator()(uint32_t w) const {
+        const uint32_t own = ties[w], next = ties[w + 1];
+        Vec<2, 0u> r;
+        r.v[0] = __builtin_popcount(tiedRows(own, next));
+        r.v[1] = largeTieRows(own, next);
         return r;
     }
 };

@@ -1,8 +1,10 @@
 """The prefix sort's arithmetic that needs no device (sadcs_amd/csrc/prefix_plan.h), compiled here and
 compared with Python's integers."""
 import os
+import random
 import subprocess
 
+import numpy as np
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "sadcs_amd", "csrc")
@@ -23,3 +25,40 @@ def test_held_bits(tmp_path, bits):
     cases = sorted({r for r in list(range(300)) + near + [2**31 - 1, 2**30, 2**31 - 257] if 0 <= r < 2**31})
     got = run_cpp(tmp_path, 'unsigned r; while (scanf("%u", &r) == 1) printf("%u\\n", heldBits(r, ' + str(bits) + "));", map(str, cases))
     assert [int(x) for x in got] == [min(r * bits, 128) for r in cases]
+
+
+def test_large_tie_rows(tmp_path):
+    """Groups of every size up to 100 rows, among them those around 24, at every place in a word."""
+    rng = random.Random(3)
+    bits, want = [], 0
+    for size in list(range(1, 101)) * 4 + [24, 25, 26] * 40 + [1] * 31 + [700, 65, 64, 33, 32]:
+        bits += [0] + [1] * (size - 1)
+        want += size if size > 24 else 0
+        gap = rng.randrange(0, 40)
+        bits += [0] * gap
+    bits += [0] * (32 - len(bits) % 32) + [0] * 32
+    words = [sum(b << r for r, b in enumerate(bits[w:w + 32])) for w in range(0, len(bits), 32)]
+    got = run_cpp(tmp_path, 'unsigned a, b, sum = 0; while (scanf("%u %u", &a, &b) == 2) sum += largeTieRows(a, b); printf("%u\\n", sum);',
+                  [f"{a} {b}" for a, b in zip(words, words[1:] + [0])])
+    assert int(got[0]) == want
+
+
+@pytest.mark.parametrize("density", [1 / 32, 1 / 96])
+@pytest.mark.parametrize("size", [2, 6, 12, 32, 64, 400])
+def test_tie_estimate(tmp_path, size, density):
+    """A sample of rows of which a share lies in groups of one size, by the sample's own counts."""
+    rng = np.random.default_rng(size)
+    rows = 1 << 20
+    for share in (0.1, 0.5, 1.0):
+        row = np.flatnonzero(rng.random(rows) < density)
+        key = np.where(row < int(rows * share / size) * size, row // size, rows + row)
+        counts = np.unique(key, return_counts=True)[1]
+        sampled, repeated, runs = (int(counts[counts >= k].sum()) for k in (1, 2, 3))
+        got = run_cpp(tmp_path, 'double s, r, u, d; while (scanf("%lf %lf %lf %lf", &s, &r, &u, &d) == 4) { TieEstimate e = estimateTies(s, r, u, d); '
+                      'printf("%.9f %.9f\\n", e.share, e.groupRows); }', [f"{sampled} {repeated} {runs} {density!r}", f"{sampled} 0 0 {density!r}", "0 0 0 0.5"])
+        got = [float(x) for x in got]
+        # Half and double of the truth: what the rules that use it leave room for. Of small groups a sample
+        # meets few rows twice; their size says only that they are small.
+        assert share / 2 <= got[0] <= min(1.0, 2 * share + 0.02) or size < 12
+        assert (size / 1.5 <= got[1] <= size * 1.5) if size >= 12 else got[1] < 24
+        assert got[2:] == [0, 1, 0, 1]
