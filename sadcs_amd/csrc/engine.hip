@@ -3061,9 +3061,16 @@ int buildWith(sadcs_ctx& ctx, const Layout& layout, const BuildRequest& rq, Text
     std::unique_ptr<Pipeline<32, Texts>> prefix;
     int status = SADCS_OK;
     bool done = false;
+    // A host call that returns the suffix array of more text than kRoomyText takes cover 32's tile merge,
+    // whose download runs while it merges: the prefix sort is over sooner and then waits for the whole
+    // download. Prefix sort and tile merge, pageable memory: 1 GiB of Markov text 176 and 168 ms, of
+    // DNA-like 195 and 174; 128 MiB 23.8 and 23.4, 25.9 and 24.4; pinned 22.7 and 21.7, 24.9 and 22.7. Below,
+    // where a kept context holds all records, 48 MiB 9.2 and 10.4, 10.2 and 11.1; the BWT alone, a fifth of
+    // the download, 1 GiB 98.6 and 128 ms. Cover 128's merge is the slower one (128 MiB 23.6 and 31.5).
+    const bool downloadsInMerge = V == 32 && job.hostSA && ctx.copyStream && layout.totalLength > kRoomyText;
     // The prefix sort, whatever the cover (it compares the few suffixes left by cover 32's sample),
     // unless merge parameters ask for the tile merge.
-    if (!job.rankOnly && !ctx.params.tiles) {
+    if (!job.rankOnly && !ctx.params.tiles && !downloadsInMerge) {
         prefix.reset(new Pipeline<32, Texts>(ctx, job, texts));
         status = prefix->runPrefix(done);
         if (done) {
