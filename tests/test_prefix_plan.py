@@ -4,7 +4,6 @@ import os
 import random
 import subprocess
 
-import numpy as np
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "sadcs_amd", "csrc")
@@ -44,21 +43,21 @@ def test_large_tie_rows(tmp_path):
 
 
 @pytest.mark.parametrize("density", [1 / 32, 1 / 96])
-@pytest.mark.parametrize("size", [2, 6, 12, 32, 64, 400])
-def test_tie_estimate(tmp_path, size, density):
-    """A sample of rows of which a share lies in groups of one size, by the sample's own counts."""
-    rng = np.random.default_rng(size)
-    rows = 1 << 20
-    for share in (0.1, 0.5, 1.0):
-        row = np.flatnonzero(rng.random(rows) < density)
-        key = np.where(row < int(rows * share / size) * size, row // size, rows + row)
-        counts = np.unique(key, return_counts=True)[1]
-        sampled, repeated, runs = (int(counts[counts >= k].sum()) for k in (1, 2, 3))
-        got = run_cpp(tmp_path, 'double s, r, u, d; while (scanf("%lf %lf %lf %lf", &s, &r, &u, &d) == 4) { TieEstimate e = estimateTies(s, r, u, d); '
-                      'printf("%.9f %.9f\\n", e.share, e.groupRows); }', [f"{sampled} {repeated} {runs} {density!r}", f"{sampled} 0 0 {density!r}", "0 0 0 0.5"])
-        got = [float(x) for x in got]
-        # Half and double of the truth: what the rules that use it leave room for. Of small groups a sample
-        # meets few rows twice; their size says only that they are small.
-        assert share / 2 <= got[0] <= min(1.0, 2 * share + 0.02) or size < 12
-        assert (size / 1.5 <= got[1] <= size * 1.5) if size >= 12 else got[1] < 24
-        assert got[2:] == [0, 1, 0, 1]
+def test_tie_estimate(tmp_path, density):
+    """Counts that a sample of this density has on average where a share of the rows lies in groups of one
+    size. A row meets the others of its group with a binomial number, of which the estimate makes a Poisson
+    number: of g rows it sees between g - 1 and g, and the share larger by as much."""
+    cases, lines = [(g, share) for g in (2, 3, 6, 12, 25, 64, 300) for share in (0.1, 0.5, 1.0)], []
+    for g, share in cases:
+        alone = (1 - density) ** (g - 1)
+        one = (g - 1) * density * (1 - density) ** (g - 2)
+        lines.append(f"1e6 {1e6 * share * (1 - alone)!r} {1e6 * share * max(0.0, 1 - alone - one)!r} {density!r}")
+    lines += [f"1000 0 0 {density!r}", f"0 0 0 {density!r}", f"1000 900 900 {density!r}"]
+    got = run_cpp(tmp_path, 'double s, r, u, d; while (scanf("%lf %lf %lf %lf", &s, &r, &u, &d) == 4) { TieEstimate e = estimateTies(s, r, u, d); '
+                  'printf("%.9f %.9f\\n", e.share, e.groupRows); }', lines)
+    got = list(zip(map(float, got[::2]), map(float, got[1::2])))
+    for (g, share), (got_share, rows) in zip(cases, got):
+        assert 0.95 * max(2, g - 1) <= rows <= 1.05 * g, (g, share)
+        assert 0.95 * share <= got_share <= min(1.0, 1.05 * share * (g - 1) / max(1, g - 2)), (g, share)
+    assert got[-3:-1] == [(0, 1), (0, 1)]
+    assert got[-1][0] == pytest.approx(0.9, rel=1e-4) and got[-1][1] == pytest.approx(1 + 12 / density, rel=1e-6)
