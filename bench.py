@@ -2,8 +2,8 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config c3] [--no-cpu]
 
-A step is one construction of the suffix array (int32) and the BWT of the whole text, in one
-merge, with the text already resident in HBM and both outputs left in HBM (the device-resident
+A step is one construction of the suffix array (int32) and the BWT of the whole text, both in one
+build, with the text already resident in HBM and both outputs left in HBM (the device-resident
 entry point of the C ABI). value = input bytes per second over the timed steps, in decimal MB/s.
 
 Printed as one JSON line, with:
@@ -15,11 +15,12 @@ Printed as one JSON line, with:
     element (list entry 4, record 44, SA 4, BWT 2), traffic its measured HBM bytes per launch
     (rocprofv3 FETCH_SIZE + WRITE_SIZE scaled by a copy of known size,
     profiles/mergeTilesKernel_c3_1GiB_traffic.md);
-  e2e_hbm_fraction: the whole step's algorithmic bytes (127.94 bytes per input byte for fused
-    SA + BWT) over the step time, against 8 TB/s;
+  e2e_hbm_fraction: 127.94 bytes per input byte over the step time, against 8 TB/s: the logical
+    traffic of the reference design for fused SA + BWT (ranking, classes, merge), a fixed yardstick
+    for every path and not the bytes that the default path moves;
   host_call: the same 1 GiB text through the host-memory API (pageable text in, SA and BWT out,
-    PCIe included), best of 3 calls, outputs compared
-    with the device-resident build's - a secondary figure, never value;
+    PCIe included; the tile merge, whose finished rows are downloaded while it runs), best of 3
+    calls, outputs compared with the device-resident build's - a secondary figure, never value;
   cpu_baseline: the reference's CPU construction (oracle/_ref, OpenMP on all host threads, cover
     128) on the same whole text, SA and BWT built separately as the reference CLI does, best of 3
     each, MB/s = n / (SA seconds + BWT seconds), with the CPU model and core count;
@@ -350,7 +351,7 @@ def host_call_measurement(ctx, text, d_sa, d_bwt, primary, runs):
     return {"value": round(n / wall / 1e6, 1), "unit": "MB/s", "ms": round(wall * 1e3, 1),
             "upload_ms": round(upload * 1e3, 1), "device_ms": round(device * 1e3, 1),
             "download_after_merge_ms": round(download * 1e3, 1), "runs": runs,
-            "io": "pageable host memory in and out over PCIe",
+            "io": "pageable host memory in and out over PCIe (cover 32: the download overlaps the top-level merge)",
             "outputs_equal_device_build": same}
 
 
@@ -545,7 +546,7 @@ def main():
         "vs_baseline": None,
         "dtype": "u8 text, u32 positions/ranks, u64 sort keys",
         "data": "synthetic",
-        "config": {"workload": f"{args.config}: {description}", "n": n, "outputs": "SA int32 + BWT, one merge",
+        "config": {"workload": f"{args.config}: {description}", "n": n, "outputs": "SA int32 + BWT, one merge" if tuned else "SA int32 + BWT, one build",
                    "cover": args.cover, "resident": "text in HBM before the timed region, outputs in HBM",
                    "merge_params": tuned or "defaults", "tuning_seconds": round(tune_seconds, 2)},
         "roofline": {"bound": "hbm", "kernel": "mergeTilesKernel (top level, SA+BWT in place)" if tuned else
@@ -555,6 +556,7 @@ def main():
                      "traffic": measured_traffic(args.config, n) if tuned and args.cover == 32 else None,  # measured at cover 32
                      "alg_bytes_per_launch": int(per_element * n), "avg_launch_ms": round(kernel * 1e3, 3)},
         "e2e_hbm_fraction": round(e2e, 4),
+        "e2e_bytes": f"{BYTES_PER_INPUT_BYTE} per input byte: the reference design's logical traffic, not this path's own",
         "phases_ms": {"ranking": round(ranking * 1e3, 2), "classes": round(classes * 1e3, 2), "merge": round(merge * 1e3, 2)},
         "peak_device_bytes_per_input_byte": round(peak_bytes / n, 3),
         "cpu_baseline": baseline,

@@ -66,8 +66,10 @@ typedef struct sadcs_stats {
 /* Construction parameters; zero fields take the defaults (of the cover, for G and tile threads). A
  * context with any of the three merge parameters set builds by the tile merge alone. Without them it
  * also builds by one workgroup a text (all texts at most 16 KiB) and by the prefix sort (most others),
- * which are faster; both order ties by cover 32 whatever the cover, and a context of one text of up
- * to 48 MiB takes 22 bytes more per input byte, where they are free, to sort it in one round. */
+ * which are faster; it keeps the tile merge for texts many of whose suffixes tie and, at cover 32, for
+ * host calls that return the suffix array of more than 48 MiB of text. The other two order ties by cover
+ * 32 whatever the cover, and a context of one text of up to 48 MiB takes 22 bytes more per input byte,
+ * where they are free, to sort it in one round. */
 typedef struct sadcs_params {
     int32_t cover;               /* 32 (default) or 128 */
     uint32_t splitter_spacing;   /* G: every G-th element of a list is a splitter; 16 (cover 32), 8 (cover 128) */

@@ -5,8 +5,9 @@
  * The tile merge (merge.h) reads one random 128-byte line per suffix and compares it three times,
  * whatever the text. Most suffixes of most texts differ within the 8 to 24 characters that fit a
  * 56-bit key, and a key read from the text in position order costs no random access at all:
- *  1. Splitters: the keys of a sample of positions, sorted; every 16th one bounds a leaf of about
- *     kLeafTarget suffixes, so leaves are even whatever the text's distribution.
+ *  1. Splitters: the keys of a sample of positions, sorted; every kOversample-th one (kCoarseOversample
+ *     of a short text) bounds a leaf of about kLeafTarget suffixes, so leaves are even whatever the
+ *     text's distribution.
  *  2. The records (key, position) are scattered into buckets straight from the text, the buckets
  *     into leaves, each time staged in LDS in bucket order so that a bucket's records leave in
  *     runs. Where memory does not hold every record, a round takes the buckets that fit and the
@@ -19,7 +20,8 @@
  *  5. Rows that tie are put in order by the difference cover's comparison. Groups of up to
  *     kTieGroupMax rows are compared in LDS; larger ones (runs, high-copy repeats) go through the
  *     tile merge as class lists of their own.
- * Texts whose suffixes tie in large groups throughout keep the tile merge alone.
+ * Texts too many of whose suffixes tie keep the tile merge alone, by what the sample shows of them: near-
+ * copies in large numbers, long runs, and ties whose lists the memory planned for the call does not hold.
  *
  * Measured against the tile merge (SA + BWT on the device): 1 GiB of Markov text 100.1 to 58.7 ms,
  * 256 MiB of DNA-like text 31.8 to 18.6 ms (cover 128: 87.2 to 18.6), 16 MiB of uniform ACGT at

@@ -16,7 +16,7 @@
  *
  * What bounds it: the barriers and LDS round trips of one workgroup's digit passes, and for a host
  * call the call's own launch and wait. Measured (host calls, SA + BWT, phases against this): 4099
- * bytes of protein 507 to 74 us; 512 documents of 200 B to 16 KiB in one batch 10.9 to 2.5 ms.
+ * bytes of protein 507 to 74 us; 512 documents of 200 B to 16 KiB in one batch 10.9 to 2.4 ms.
  */
 #pragma once
 
@@ -27,9 +27,10 @@
 namespace sadcs {
 
 // The largest text whose arrays fit the LDS of a CU beside the counters: 16384 bytes take 127 KB of
-// 160. Alone at that size, against the prefix sort: protein-like 0.14 to 0.19 ms, DNA-like 0.47 to
-// 0.52, periodic 0.44 to 1.19, but Markov 0.53 to 0.30 (8192 bytes: 0.30 to 0.27); what a text is like
-// is not known here, and a batch of such texts has a workgroup for each.
+// 160. Alone at that size, from host memory, against a byte more by the prefix sort: protein-like 0.14 and
+// 0.24 ms, DNA-like 0.44 and 0.53, periodic 0.45 and 0.66, but Markov 0.57 and 0.33; what a text is like is
+// not known here, and a batch of such texts has a workgroup for each (4096 of Markov text 2.4 ms, by the tile
+// merge 6.9).
 constexpr uint32_t kSmallMax = 16384;
 constexpr int kSmallBins = 256;
 
